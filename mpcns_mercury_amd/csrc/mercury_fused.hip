@@ -506,14 +506,17 @@ __global__ void __launch_bounds__(256) k_rhs_tile(const MercRange R, const MercB
 // PV_s, U+ (Tools.cpp:159-301), Hall E_hc and beta (Hall.cpp:87-124), the
 // contravariant velocity of U+ per axis (cell_u_contra, Ideal.cpp:513-526) and,
 // on owned cells when requested, the CFL candidate of Compute_Timestep.
-// Six waves per SIMD: the FP64 body fits in 80 VGPRs without spilling (102
-// unconstrained, four waves), and the latency-bound pass runs 10 % faster
-// (398 -> 359 us on shell6); seven waves would spill.
+// Bound by FP64 arithmetic at its occupancy (VALU issue about half of the time)
+// since every array is read once: 1.30 -> 0.83 GB fetched per launch on the six
+// sectors of 2.53 M cells (28 arrays of the 3.59 M-point box, as counted), 342 ->
+// 326 us FP64 and 261 -> 243 us mixed.  Waves per SIMD: what the body fits
+// without spilling, four in FP64 (five and six spill: 474 us), six in the mixed
+// form with two species, four with three.
 // ENS: an ensemble context (per-block Hall coefficient and per-run dt); a
 // one-run context takes both from the kernel arguments and keeps every
 // register of the six-wave budget for the body.
 template <bool MIX, int NS, bool ENS>
-__global__ void __attribute__((amdgpu_waves_per_eu(NS == 2 ? 6 : 5))) k_cell_end(const MercRange R, const MercBlk *__restrict__ B, double *const *__restrict__ F_,
+__global__ void __attribute__((amdgpu_waves_per_eu(MIX ? (NS == 2 ? 6 : 4) : 4))) k_cell_end(const MercRange R, const MercBlk *__restrict__ B, double *const *__restrict__ F_,
                            const float *const *__restrict__ G_, const MercPhys P, unsigned long long *__restrict__ dt_bits,
                            int compute_dt) {
     gdouble *const *__restrict__ F = gslots(F_);
@@ -526,114 +529,130 @@ __global__ void __attribute__((amdgpu_waves_per_eu(NS == 2 ? 6 : 5))) k_cell_end
     if (located) {
         const MercBlk &bk = B[p.b];
         const long long q = p.q;
-        double pv[NS][5];
+        // Each array is read once: the slots may alias for all the compiler
+        // knows, so a value read on both sides of a store is loaded twice.  The
+        // pass goes in two halves (the state's own values, then the faces), each
+        // with its stores at its end: in one piece it does not fit its registers.
+        double U[NS][5], pv[NS][5], r[NS];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int c = 0; c < 5; ++c) U[s][c] = F[SPEC_U(s) + c][q];
+        const double Bx = F[SL_BC][q], By = F[SL_BC + 1][q], Bz = F[SL_BC + 2][q];
+        const double jac = fabs(F[SL_JAC][q]);
+        T hc[4];
+        double up[3];
+#pragma unroll
         for (int s = 0; s < NS; ++s) {
-            const int su = SPEC_U(s);
             const double coeff = species_coeff(P, s);
-            const double rho = dmax(F[su][q], 1e-12);
-            const double u = F[su + 1][q] / rho, v = F[su + 2][q] / rho, w = F[su + 3][q] / rho;
-            const double E = F[su + 4][q];
+            const double rho = dmax(U[s][0], 1e-12);
+            const double u = U[s][1] / rho, v = U[s][2] / rho, w = U[s][3] / rho;
             const double ke = 0.5 * rho * (u * u + v * v + w * w);
-            double eint = E - ke;
+            double eint = U[s][4] - ke;
             if (eint < 0.0) eint = 0.0;
             double pr = (P.gamma - 1.0) * eint;
             pr = dmax(pr, 1e-12);
             pv[s][0] = u; pv[s][1] = v; pv[s][2] = w; pv[s][3] = pr; pv[s][4] = pr / (rho * coeff);
-            const int sp = SPEC_PV(s);
+            r[s] = dmax(U[s][0], 0.0);
+        }
+        {
+            // one limiter serves U+ (floored densities) and the Hall terms (raw
+            // densities, Hall.cpp:92-95): it floors its inputs at 0 itself
+            const Num n = num_limiter(P, r[0], r[1], NS > 2 ? r[NS - 1] : 0.0, NS);
+            for (int c = 0; c < 3; ++c) {
+                const double uH = (r[0] > 1e-20) ? pv[0][c] : 0.0;
+                const double uN = (r[1] > 1e-20) ? pv[1][c] : 0.0;
+                up[c] = n.chi[0] * uH + n.chi[1] * uN;
+                if constexpr (NS > 2) up[c] = up[c] + n.chi[2] * ((r[2] > 1e-20) ? pv[2][c] : 0.0);
+            }
+            const T alpha = (T)((ENS ? bk.hall_coef : P.hall_coef) / n.ne_eff);
+            const T Jx = (T)F[SL_JC][q], Jy = (T)F[SL_JC + 1][q], Jz = (T)F[SL_JC + 2][q];
+            const T bx = (T)Bx, by = (T)By, bz = (T)Bz;
+            hc[0] = alpha * (Jy * bz - Jz * by), hc[1] = alpha * (Jz * bx - Jx * bz), hc[2] = alpha * (Jx * by - Jy * bx);
+            hc[3] = fabs(alpha) * PR::sq(bx * bx + by * by + bz * bz);
+        }
+        // contravariant velocities (need the face of the next index on each axis)
+        // and the time-step candidate on owned cells
+        const int idx[3] = {p.i, p.j, p.k};
+        const T inv_jac = (T)(1.0 / (jac + 1.0e-30));
+        const bool cand = compute_dt && p.i >= 0 && p.j >= 0 && p.k >= 0 && p.i < bk.m[0] && p.j < bk.m[1] && p.k < bk.m[2] && !(jac <= 0.0);
+        // per species state first, then one pass over the six faces: the face
+        // normal and |S| (the stored area, bitwise the same sqrt) are shared by
+        // the species.  FP64 in the FP64 forms; the mixed form evaluates the
+        // candidate in FP32 (the global minimum stays an exact reduction of FP64
+        // values)
+        const T bx = (T)Bx, by = (T)By, bz = (T)Bz, gam = (T)P.gamma, mi = (T)P.inver_MA2;
+        const T B2 = bx * bx + by * by + bz * bz;
+        T rho[NS], ux[NS], uy[NS], uz[NS], cs2[NS], vA2[NS], denom[NS];
+        if (cand) {
+#pragma unroll
+            for (int s = 0; s < NS; ++s) {
+                denom[s] = T(0);
+                rho[s] = tmax((T)U[s][0], T(1e-2));
+                ux[s] = PR::div((T)U[s][1], rho[s]);
+                uy[s] = PR::div((T)U[s][2], rho[s]);
+                uz[s] = PR::div((T)U[s][3], rho[s]);
+                const T ke = T(0.5) * rho[s] * (ux[s] * ux[s] + uy[s] * uy[s] + uz[s] * uz[s]);
+                const T pr = (gam - T(1)) * ((T)U[s][4] - ke);
+                cs2[s] = PR::div(gam * pr, rho[s]);
+                vA2[s] = PR::div(mi * B2, rho[s]);
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
             for (int c = 0; c < 5; ++c) {
+                const int sp = SPEC_PV(s);
                 if (c == 3) F[sp + 3][q] = pv[s][3];
                 else wr<MIX>(F, G, sp + c, q, pv[s][c]);
             }
-        }
-        double r[NS];
-        for (int s = 0; s < NS; ++s) r[s] = dmax(F[SPEC_U(s)][q], 0.0);
-        // one limiter serves U+ (floored densities) and the Hall terms (raw
-        // densities, Hall.cpp:92-95): it floors its inputs at 0 itself
-        const Num n = num_limiter(P, r[0], r[1], NS > 2 ? r[NS - 1] : 0.0, NS);
-        double up[3];
         for (int c = 0; c < 3; ++c) {
-            const double uH = (r[0] > 1e-20) ? pv[0][c] : 0.0;
-            const double uN = (r[1] > 1e-20) ? pv[1][c] : 0.0;
-            up[c] = n.chi[0] * uH + n.chi[1] * uN;
-            if constexpr (NS > 2) up[c] = up[c] + n.chi[2] * ((r[2] > 1e-20) ? pv[2][c] : 0.0);
             wr<MIX>(F, G, SL_UP + c, q, up[c]);
+            wr<MIX>(F, G, SL_EHC + c, q, hc[c]);
         }
-        const Num &nh = n;
-        const double Bx = F[SL_BC][q], By = F[SL_BC + 1][q], Bz = F[SL_BC + 2][q];
-        {
-            const T alpha = (T)((ENS ? bk.hall_coef : P.hall_coef) / nh.ne_eff);
-            const T Jx = (T)F[SL_JC][q], Jy = (T)F[SL_JC + 1][q], Jz = (T)F[SL_JC + 2][q];
-            const T bx = (T)Bx, by = (T)By, bz = (T)Bz;
-            const T e0 = alpha * (Jy * bz - Jz * by), e1 = alpha * (Jz * bx - Jx * bz), e2 = alpha * (Jx * by - Jy * bx);
-            const T hb = fabs(alpha) * PR::sq(bx * bx + by * by + bz * bz);
-            wr<MIX>(F, G, SL_EHC, q, e0);
-            wr<MIX>(F, G, SL_EHC + 1, q, e1);
-            wr<MIX>(F, G, SL_EHC + 2, q, e2);
-            wr<MIX>(F, G, SL_HB, q, hb);
-        }
-        // contravariant velocities (need the face of the next index on each axis)
-        const int idx[3] = {p.i, p.j, p.k};
-        const T inv_jac = MIX ? (T)(1.0 / (fabs(F[SL_JAC][q]) + 1.0e-30)) : (T)(1.0 / (fabs(F[SL_JAC][q]) + 1.0e-30));
+        wr<MIX>(F, G, SL_HB, q, hc[3]);
+        T ucon[3];
+#pragma unroll
         for (int a = 0; a < 3; ++a) {
-            if (idx[a] + 1 > bk.m[a] + bk.g) continue;
-            const long long cp = q + AX(p, a);
+            // the upper face of the last ghost cell is not in the box: that
+            // value is not stored, and its face is read at the cell itself
+            const long long cp = idx[a] + 1 > bk.m[a] + bk.g ? q : q + AX(p, a);
             const int s0 = SL_JD + 3 * a;
-            const T kx = T(0.5) * ((T)F[s0][q] + (T)F[s0][cp]);
-            const T ky = T(0.5) * ((T)F[s0 + 1][q] + (T)F[s0 + 1][cp]);
-            const T kz = T(0.5) * ((T)F[s0 + 2][q] + (T)F[s0 + 2][cp]);
-            wr<MIX>(F, G, SL_UCON + a, q, (kx * (T)up[0] + ky * (T)up[1] + kz * (T)up[2]) * inv_jac);
-        }
-        // time-step candidate on owned cells
-        if (compute_dt && p.i >= 0 && p.j >= 0 && p.k >= 0 && p.i < bk.m[0] && p.j < bk.m[1] && p.k < bk.m[2]) {
-            const double V = fabs(F[SL_JAC][q]);
-            if (!(V <= 0.0)) {
-                // per species state first, then one pass over the six faces:
-                // the face normal and |S| (the stored area, bitwise the same
-                // sqrt) are shared by the species.  FP64 in the FP64 forms; the
-                // mixed form evaluates the candidate in FP32 (the global minimum
-                // stays an exact reduction of FP64 values)
-                const T bx = (T)Bx, by = (T)By, bz = (T)Bz, gam = (T)P.gamma, mi = (T)P.inver_MA2;
-                const T B2 = bx * bx + by * by + bz * bz;
-                T rho[NS], ux[NS], uy[NS], uz[NS], cs2[NS], vA2[NS], denom[NS];
-                for (int s = 0; s < NS; ++s) {
-                    const int su = SPEC_U(s);
-                    denom[s] = T(0);
-                    rho[s] = tmax((T)F[su][q], T(1e-2));
-                    ux[s] = PR::div((T)F[su + 1][q], rho[s]);
-                    uy[s] = PR::div((T)F[su + 2][q], rho[s]);
-                    uz[s] = PR::div((T)F[su + 3][q], rho[s]);
-                    const T E = (T)F[su + 4][q];
-                    const T ke = T(0.5) * rho[s] * (ux[s] * ux[s] + uy[s] * uy[s] + uz[s] * uz[s]);
-                    const T pr = (gam - T(1)) * (E - ke);
-                    cs2[s] = PR::div(gam * pr, rho[s]);
-                    vA2[s] = PR::div(mi * B2, rho[s]);
-                }
-                for (int a = 0; a < 3; ++a)
-                    for (int sd = 0; sd < 2; ++sd) {
-                        const long long fq = q + (sd ? AX(p, a) : 0LL);
-                        const T ax = (T)F[SL_JD + 3 * a][fq], ay = (T)F[SL_JD + 3 * a + 1][fq], az = (T)F[SL_JD + 3 * a + 2][fq];
-                        const T A = st<MIX>(F, G, SL_AREA + a, fq);
-                        if (A <= T(0)) {
-                            for (int s = 0; s < NS; ++s) denom[s] += T(0);
-                            continue;
-                        }
-                        T nx = PR::div(ax, A), ny = PR::div(ay, A), nz = PR::div(az, A);
-                        if (!sd) { nx = -nx; ny = -ny; nz = -nz; }
-                        const T Bn = bx * nx + by * ny + bz * nz;
-                        for (int s = 0; s < NS; ++s) {
-                            const T un = ux[s] * nx + uy[s] * ny + uz[s] * nz;
-                            const T vAn2 = PR::div(mi * (Bn * Bn), rho[s]);
-                            const T t = cs2[s] + vA2[s];
-                            T disc = t * t - T(4) * cs2[s] * vAn2;
-                            if (disc < T(0)) disc = T(0);
-                            const T cf = PR::sq(T(0.5) * (t + PR::sq(disc)));
-                            denom[s] += (fabs(un) + cf) * A;
-                        }
+            const T S[2][3] = {{(T)F[s0][q], (T)F[s0 + 1][q], (T)F[s0 + 2][q]}, {(T)F[s0][cp], (T)F[s0 + 1][cp], (T)F[s0 + 2][cp]}};
+            const T kx = T(0.5) * (S[0][0] + S[1][0]);
+            const T ky = T(0.5) * (S[0][1] + S[1][1]);
+            const T kz = T(0.5) * (S[0][2] + S[1][2]);
+            ucon[a] = (kx * (T)up[0] + ky * (T)up[1] + kz * (T)up[2]) * inv_jac;
+            if (cand) {
+#pragma unroll
+                for (int sd = 0; sd < 2; ++sd) {
+                    const T ax = S[sd][0], ay = S[sd][1], az = S[sd][2];
+                    const T A = st<MIX>(F, G, SL_AREA + a, sd ? cp : q);
+                    if (A <= T(0)) {
+                        for (int s = 0; s < NS; ++s) denom[s] += T(0);
+                        continue;
                     }
-                for (int s = 0; s < NS; ++s)
-                    if (denom[s] > T(0)) best = dmin(best, P.cfl * V / (double)denom[s]);
+                    T nx = PR::div(ax, A), ny = PR::div(ay, A), nz = PR::div(az, A);
+                    if (!sd) { nx = -nx; ny = -ny; nz = -nz; }
+                    const T Bn = bx * nx + by * ny + bz * nz;
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) {
+                        const T un = ux[s] * nx + uy[s] * ny + uz[s] * nz;
+                        const T vAn2 = PR::div(mi * (Bn * Bn), rho[s]);
+                        const T t = cs2[s] + vA2[s];
+                        T disc = t * t - T(4) * cs2[s] * vAn2;
+                        if (disc < T(0)) disc = T(0);
+                        const T cf = PR::sq(T(0.5) * (t + PR::sq(disc)));
+                        denom[s] += (fabs(un) + cf) * A;
+                    }
+                }
             }
         }
+        if (cand)
+            for (int s = 0; s < NS; ++s)
+                if (denom[s] > T(0)) best = dmin(best, P.cfl * jac / (double)denom[s]);
+        for (int c = 0; c < 3; ++c)
+            if (idx[c] + 1 <= bk.m[c] + bk.g) wr<MIX>(F, G, SL_UCON + c, q, ucon[c]);
     }
     if (!compute_dt) return;
     // the run is read here, not before the body: its register is not held across it
@@ -661,7 +680,10 @@ DEVI typename Prec<MIX>::T emf_flux_u(gdouble *const *__restrict__ F, const gflo
 // term, the node electron pressure its edges need: the mean of p_H + p_Na over
 // the 8 cells around the node, summed in the order of AddAmbipolarEdgeEMF_
 // (MercurySolver_MagExplicit_Ambipo.cpp:3-143), once per node instead of once
-// per edge end
+// per edge end.  68 loads per point, each made once (84 when every face loaded
+// its own): 180 -> 160 us FP64 and 139 -> 128 us mixed on the six sectors of
+// 2.53 M cells; held to four waves and bound by address work (forced to six waves
+// it spills, 328 us).
 template <bool MIX>
 __global__ void k_eface_u(const MercRange R, const MercBlk *__restrict__ B, double *const *__restrict__ F_,
                           const float *const *__restrict__ G_, int ambi, int ns) {
@@ -671,9 +693,13 @@ __global__ void k_eface_u(const MercRange R, const MercBlk *__restrict__ B, doub
     LOCATE(R);
     const MercBlk &bk = B[p.b];
     const int idx[3] = {p.i, p.j, p.k};
-    if (ambi && p.i >= 0 && p.j >= 0 && p.k >= 0 && p.i <= bk.m[0] && p.j <= bk.m[1] && p.k <= bk.m[2]) {
+    const bool node = ambi && p.i >= 0 && p.j >= 0 && p.k >= 0 && p.i <= bk.m[0] && p.j <= bk.m[1] && p.k <= bk.m[2];
+    // the values are stored after every load of the point: the slots may alias
+    // for all the compiler knows, and it would load B and U_con again behind
+    // each store
+    T sum = T(0);
+    if (node) {
         const long long di = OI(p), dj = OJ(p);
-        T sum = T(0);
         for (int ddi = -1; ddi <= 0; ++ddi)
             for (int ddj = -1; ddj <= 0; ++ddj)
                 for (int ddk = -1; ddk <= 0; ++ddk) {
@@ -682,38 +708,42 @@ __global__ void k_eface_u(const MercRange R, const MercBlk *__restrict__ B, doub
                     if (ns > 2) pe = pe + (T)F[SL_PVHE + 3][c];
                     sum += pe;
                 }
-        wr<MIX>(F, G, SL_PEN, p.q, T(0.125) * sum);
     }
+    // per face axis: the transport of the two tangential B fluxes.  Only the
+    // two tangential components are written: the normal one is zero by
+    // construction (the per-function pass stores that zero) and its slot keeps
+    // the zero of the arena's initialisation
+    // (the faces at the ends of the range are computed too and not stored: with
+    // two ghost layers their reads stay in the box, and the loads that the three
+    // faces share are made once)
+    bool ok[3];
+    T g1[3], g2[3];
+#pragma unroll
     for (int fa = 0; fa < 3; ++fa) {
-        bool ok = true;
+        ok[fa] = true;
         for (int a = 0; a < 3; ++a) {
             const int ohi = bk.m[a] + (a == fa ? 1 : 0);
             const int lo = (-1 > -bk.g + 1) ? -1 : -bk.g + 1;
             const int hi = (ohi + 1 < ohi + bk.g - 1) ? ohi + 1 : ohi + bk.g - 1;
-            if (idx[a] < lo || idx[a] >= hi) ok = false;
+            if (idx[a] < lo || idx[a] >= hi) ok[fa] = false;
         }
-        if (!ok) continue;
         const long long Rq = p.q, Lq = p.q - AX(p, fa);
         const T bff = (T)F[SL_B + fa][Rq] + (T)F[SL_BADD + fa][Rq];
-        // only the two tangential components are written: the normal one is
-        // zero by construction (the per-function pass stores that zero) and
-        // its slot keeps the zero of the arena's initialisation
-        if (fa == 0) {
-            const T Gex = emf_flux_u<MIX>(F, G, p, 1, 0, Lq, Rq, bff);
-            const T Gzx = emf_flux_u<MIX>(F, G, p, 2, 0, Lq, Rq, bff);
-            wr<MIX>(F, G, SL_EF + 1, Rq, Gzx);
-            wr<MIX>(F, G, SL_EF + 2, Rq, -Gex);
-        } else if (fa == 1) {
-            const T Gxe = emf_flux_u<MIX>(F, G, p, 0, 1, Lq, Rq, bff);
-            const T Gze = emf_flux_u<MIX>(F, G, p, 2, 1, Lq, Rq, bff);
-            wr<MIX>(F, G, SL_EF + 3, Rq, -Gze);
-            wr<MIX>(F, G, SL_EF + 5, Rq, Gxe);
-        } else {
-            const T Gxz = emf_flux_u<MIX>(F, G, p, 0, 2, Lq, Rq, bff);
-            const T Gez = emf_flux_u<MIX>(F, G, p, 1, 2, Lq, Rq, bff);
-            wr<MIX>(F, G, SL_EF + 6, Rq, Gez);
-            wr<MIX>(F, G, SL_EF + 7, Rq, -Gxz);
-        }
+        g1[fa] = emf_flux_u<MIX>(F, G, p, fa == 0 ? 1 : 0, fa, Lq, Rq, bff);
+        g2[fa] = emf_flux_u<MIX>(F, G, p, fa == 2 ? 1 : 2, fa, Lq, Rq, bff);
+    }
+    if (node) wr<MIX>(F, G, SL_PEN, p.q, T(0.125) * sum);
+    if (ok[0]) {
+        wr<MIX>(F, G, SL_EF + 1, p.q, g2[0]);
+        wr<MIX>(F, G, SL_EF + 2, p.q, -g1[0]);
+    }
+    if (ok[1]) {
+        wr<MIX>(F, G, SL_EF + 3, p.q, -g2[1]);
+        wr<MIX>(F, G, SL_EF + 5, p.q, g1[1]);
+    }
+    if (ok[2]) {
+        wr<MIX>(F, G, SL_EF + 6, p.q, g2[2]);
+        wr<MIX>(F, G, SL_EF + 7, p.q, -g1[2]);
     }
 }
 
@@ -751,35 +781,39 @@ __global__ void k_edge_total(const MercRange R, const MercBlk *__restrict__ B, d
     const bool local = P.local_enabled != 0.0 && P.local_eta_max > 0.0 && P.local_r_decay > 0.0;
 #define FB(s, o) ((T)F[(s)][q + (o)])
 #define FE(s, o) (st<MIX>(F, G, (s), q + (o)))
-    for (int a = 0; a < 3; ++a) {
-        if (idx[a] >= bk.m[a]) continue;
-        T E;
-        if (a == 0) {
-            const T Ec = T(0.25) * (FE(SL_EF + 3, 0) + FE(SL_EF + 3, -dk) + FE(SL_EF + 6, 0) + FE(SL_EF + 6, -dj));
-            const T ae = maxu4_p<MIX>(F, G, 1, q, q - dj, q - dk, q - dj - dk);
-            const T az = maxu4_p<MIX>(F, G, 2, q, q - dj, q - dk, q - dj - dk);
-            const T dBz = FB(SL_B + 2, 0) - FB(SL_B + 2, -dj);
-            const T dBe = FB(SL_B + 1, 0) - FB(SL_B + 1, -dk);
-            E = Ec + Cuct * (T(0.5) * ae * dBz - T(0.5) * az * dBe);
-        } else if (a == 1) {
-            const T Ec = T(0.25) * (FE(SL_EF + 1, 0) + FE(SL_EF + 1, -dk) + FE(SL_EF + 7, 0) + FE(SL_EF + 7, -di));
-            const T az = maxu4_p<MIX>(F, G, 2, q, q - di, q - dk, q - di - dk);
-            const T ax = maxu4_p<MIX>(F, G, 0, q, q - di, q - dk, q - di - dk);
-            const T dBx = FB(SL_B + 0, 0) - FB(SL_B + 0, -dk);
-            const T dBz = FB(SL_B + 2, 0) - FB(SL_B + 2, -di);
-            E = Ec + Cuct * (T(0.5) * az * dBx - T(0.5) * ax * dBz);
-        } else {
-            const T Ec = T(0.25) * (FE(SL_EF + 2, 0) + FE(SL_EF + 2, -dj) + FE(SL_EF + 5, 0) + FE(SL_EF + 5, -di));
-            const T ax = maxu4_p<MIX>(F, G, 0, q, q - di, q - dj, q - di - dj);
-            const T ae = maxu4_p<MIX>(F, G, 1, q, q - di, q - dj, q - di - dj);
-            const T dBe = FB(SL_B + 1, 0) - FB(SL_B + 1, -di);
-            const T dBx = FB(SL_B + 0, 0) - FB(SL_B + 0, -dj);
-            E = Ec + Cuct * (T(0.5) * ax * dBe - T(0.5) * ae * dBx);
-        }
-        if (ambi) {
-            const long long ea = AX(p, a);
-            const T pe[2] = {st<MIX>(F, G, SL_PEN, q), st<MIX>(F, G, SL_PEN, q + ea)};  // node electron pressure (k_eface_u)
-            const int ns = nspec(P);
+    // Every edge of the point is computed, also the one past an upper face whose
+    // value is not stored (its reads stay in the box), term by term and not edge
+    // by edge, and everything is stored at the end: the loads that the three
+    // edges share then sit in one block with no store between them, and each is
+    // made once (115 per point and not 155).
+    T E[3], hall[3];
+    const T dB0j = FB(SL_B + 0, 0) - FB(SL_B + 0, -dj), dB0k = FB(SL_B + 0, 0) - FB(SL_B + 0, -dk);
+    const T dB1i = FB(SL_B + 1, 0) - FB(SL_B + 1, -di), dB1k = FB(SL_B + 1, 0) - FB(SL_B + 1, -dk);
+    const T dB2i = FB(SL_B + 2, 0) - FB(SL_B + 2, -di), dB2j = FB(SL_B + 2, 0) - FB(SL_B + 2, -dj);
+    {
+        const T Ec = T(0.25) * (FE(SL_EF + 3, 0) + FE(SL_EF + 3, -dk) + FE(SL_EF + 6, 0) + FE(SL_EF + 6, -dj));
+        const T ae = maxu4_p<MIX>(F, G, 1, q, q - dj, q - dk, q - dj - dk);
+        const T az = maxu4_p<MIX>(F, G, 2, q, q - dj, q - dk, q - dj - dk);
+        E[0] = Ec + Cuct * (T(0.5) * ae * dB2j - T(0.5) * az * dB1k);
+    }
+    {
+        const T Ec = T(0.25) * (FE(SL_EF + 1, 0) + FE(SL_EF + 1, -dk) + FE(SL_EF + 7, 0) + FE(SL_EF + 7, -di));
+        const T az = maxu4_p<MIX>(F, G, 2, q, q - di, q - dk, q - di - dk);
+        const T ax = maxu4_p<MIX>(F, G, 0, q, q - di, q - dk, q - di - dk);
+        E[1] = Ec + Cuct * (T(0.5) * az * dB0k - T(0.5) * ax * dB2i);
+    }
+    {
+        const T Ec = T(0.25) * (FE(SL_EF + 2, 0) + FE(SL_EF + 2, -dj) + FE(SL_EF + 5, 0) + FE(SL_EF + 5, -di));
+        const T ax = maxu4_p<MIX>(F, G, 0, q, q - di, q - dj, q - di - dj);
+        const T ae = maxu4_p<MIX>(F, G, 1, q, q - di, q - dj, q - di - dj);
+        E[2] = Ec + Cuct * (T(0.5) * ax * dB1i - T(0.5) * ae * dB0j);
+    }
+    if (ambi) {
+        const T pe = st<MIX>(F, G, SL_PEN, q);  // node electron pressure (k_eface_u)
+        const int ns = nspec(P);
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            const T pe1 = st<MIX>(F, G, SL_PEN, q + AX(p, a));
             double rH = 0.0, rN = 0.0, rHe = 0.0;
             const long long t1 = (a == 0) ? dj : di, t2 = (a == 2) ? dj : 1;
             for (int d1 = -1; d1 <= 0; ++d1)
@@ -790,9 +824,12 @@ __global__ void k_edge_total(const MercRange R, const MercBlk *__restrict__ B, d
                     if (ns > 2) rHe += F[SL_UHE][c];
                 }
             const Num n = num_limiter(P, 0.25 * rH, 0.25 * rN, 0.25 * rHe, ns);
-            E -= PR::div((T)P.pressure_coef * (pe[1] - pe[0]), (T)n.ne_eff);
+            E[a] -= PR::div((T)P.pressure_coef * (pe1 - pe), (T)n.ne_eff);
         }
-        if (arti) {
+    }
+    if (arti) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
             const T J1 = FB(SL_J + a, 0);
             const T dx = st<MIX>(F, G, SL_DR + 3 * a, q), dy = st<MIX>(F, G, SL_DR + 3 * a + 1, q), dz = st<MIX>(F, G, SL_DR + 3 * a + 2, q);
             const T drl = PR::sq(dx * dx + dy * dy + dz * dz);
@@ -805,74 +842,76 @@ __global__ void k_edge_total(const MercRange R, const MercBlk *__restrict__ B, d
                 qq = tmax(T(0), tmin(T(1), qq));
                 eta = (T)P.arti_eta_max * (qq * qq * (T(3) - T(2) * qq));
             }
-            E += eta * J1;
+            E[a] += eta * J1;
         }
-        if (local) E += st<MIX>(F, G, SL_LETA + a, q) * FB(SL_J + a, 0);
-        if (!with_hall) {
-            F[SL_E + a][q] = (double)E;
-            continue;
-        }
-        // Hall EMF of this edge (Hall.cpp:126-385)
+    }
+    if (local)
+#pragma unroll
+        for (int a = 0; a < 3; ++a) E[a] += st<MIX>(F, G, SL_LETA + a, q) * FB(SL_J + a, 0);
+    if (with_hall) {
+        // Hall EMF (Hall.cpp:126-385)
         const T eps = T(1e-14), Cwh = T(0.1);
-        long long c[4];
-        if (a == 0) { c[0] = q - dj - dk; c[1] = q - dj; c[2] = q - dk; c[3] = q; }
-        else if (a == 1) { c[0] = q - di - dk; c[1] = q - di; c[2] = q - dk; c[3] = q; }
-        else { c[0] = q - di - dj; c[1] = q - di; c[2] = q - dj; c[3] = q; }
-        T Ecc[3];
-        for (int d = 0; d < 3; ++d)
-            Ecc[d] = T(0.25) * (st<MIX>(F, G, SL_EHC + d, c[0]) + st<MIX>(F, G, SL_EHC + d, c[1]) + st<MIX>(F, G, SL_EHC + d, c[2]) +
-                                st<MIX>(F, G, SL_EHC + d, c[3]));
-        const T Ecen = Ecc[0] * st<MIX>(F, G, SL_DR + 3 * a, q) + Ecc[1] * st<MIX>(F, G, SL_DR + 3 * a + 1, q) +
-                       Ecc[2] * st<MIX>(F, G, SL_DR + 3 * a + 2, q);
-        const T be = tmax(tmax(st<MIX>(F, G, SL_HB, c[0]), st<MIX>(F, G, SL_HB, c[1])), tmax(st<MIX>(F, G, SL_HB, c[2]), st<MIX>(F, G, SL_HB, c[3])));
-        const T L = tmax(st<MIX>(F, G, SL_DL + a, q), eps);
 #define AR(s, o) st<MIX>(F, G, (s), q + (o))
-        T val;
-        if (a == 0) {
-            const T Az = T(0.5) * (AR(SL_AREA + 2, 0) + AR(SL_AREA + 2, -dj));
-            const T ihe = PR::div(L, tmax(Az, eps));
-            const T mue = Cwh * be * ihe * ihe;
-            const T Ae = T(0.5) * (AR(SL_AREA + 1, 0) + AR(SL_AREA + 1, -dk));
-            const T ihz = PR::div(L, tmax(Ae, eps));
-            const T muz = Cwh * be * ihz * ihz;
-            const T d1 = FB(SL_B + 2, 0) - FB(SL_B + 2, -dj);
-            const T d2 = FB(SL_B + 1, 0) - FB(SL_B + 1, -dk);
-            val = Ecen + T(0.5) * mue * d1 - T(0.5) * muz * d2;
-        } else if (a == 1) {
-            const T Ax = T(0.5) * (AR(SL_AREA + 0, 0) + AR(SL_AREA + 0, -dk));
-            const T ihz = PR::div(L, tmax(Ax, eps));
-            const T muz = Cwh * be * ihz * ihz;
-            const T Az = T(0.5) * (AR(SL_AREA + 2, 0) + AR(SL_AREA + 2, -di));
-            const T ihx = PR::div(L, tmax(Az, eps));
-            const T mux = Cwh * be * ihx * ihx;
-            const T d1 = FB(SL_B + 0, 0) - FB(SL_B + 0, -dk);
-            const T d2 = FB(SL_B + 2, 0) - FB(SL_B + 2, -di);
-            val = Ecen + T(0.5) * muz * d1 - T(0.5) * mux * d2;
-        } else {
-            const T Ae = T(0.5) * (AR(SL_AREA + 1, 0) + AR(SL_AREA + 1, -di));
-            const T ihx = PR::div(L, tmax(Ae, eps));
-            const T mux = Cwh * be * ihx * ihx;
-            const T Ax = T(0.5) * (AR(SL_AREA + 0, 0) + AR(SL_AREA + 0, -dj));
-            const T ihe = PR::div(L, tmax(Ax, eps));
-            const T mue = Cwh * be * ihe * ihe;
-            const T d1 = FB(SL_B + 1, 0) - FB(SL_B + 1, -di);
-            const T d2 = FB(SL_B + 0, 0) - FB(SL_B + 0, -dj);
-            val = Ecen + T(0.5) * mux * d1 - T(0.5) * mue * d2;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            long long c[4];
+            if (a == 0) { c[0] = q - dj - dk; c[1] = q - dj; c[2] = q - dk; c[3] = q; }
+            else if (a == 1) { c[0] = q - di - dk; c[1] = q - di; c[2] = q - dk; c[3] = q; }
+            else { c[0] = q - di - dj; c[1] = q - di; c[2] = q - dj; c[3] = q; }
+            T Ecc[3];
+            for (int d = 0; d < 3; ++d)
+                Ecc[d] = T(0.25) * (st<MIX>(F, G, SL_EHC + d, c[0]) + st<MIX>(F, G, SL_EHC + d, c[1]) + st<MIX>(F, G, SL_EHC + d, c[2]) +
+                                    st<MIX>(F, G, SL_EHC + d, c[3]));
+            const T Ecen = Ecc[0] * st<MIX>(F, G, SL_DR + 3 * a, q) + Ecc[1] * st<MIX>(F, G, SL_DR + 3 * a + 1, q) +
+                           Ecc[2] * st<MIX>(F, G, SL_DR + 3 * a + 2, q);
+            const T be = tmax(tmax(st<MIX>(F, G, SL_HB, c[0]), st<MIX>(F, G, SL_HB, c[1])), tmax(st<MIX>(F, G, SL_HB, c[2]), st<MIX>(F, G, SL_HB, c[3])));
+            const T L = tmax(st<MIX>(F, G, SL_DL + a, q), eps);
+            T val;
+            if (a == 0) {
+                const T Az = T(0.5) * (AR(SL_AREA + 2, 0) + AR(SL_AREA + 2, -dj));
+                const T ihe = PR::div(L, tmax(Az, eps));
+                const T mue = Cwh * be * ihe * ihe;
+                const T Ae = T(0.5) * (AR(SL_AREA + 1, 0) + AR(SL_AREA + 1, -dk));
+                const T ihz = PR::div(L, tmax(Ae, eps));
+                const T muz = Cwh * be * ihz * ihz;
+                val = Ecen + T(0.5) * mue * dB2j - T(0.5) * muz * dB1k;
+            } else if (a == 1) {
+                const T Ax = T(0.5) * (AR(SL_AREA + 0, 0) + AR(SL_AREA + 0, -dk));
+                const T ihz = PR::div(L, tmax(Ax, eps));
+                const T muz = Cwh * be * ihz * ihz;
+                const T Az = T(0.5) * (AR(SL_AREA + 2, 0) + AR(SL_AREA + 2, -di));
+                const T ihx = PR::div(L, tmax(Az, eps));
+                const T mux = Cwh * be * ihx * ihx;
+                val = Ecen + T(0.5) * muz * dB0k - T(0.5) * mux * dB2i;
+            } else {
+                const T Ae = T(0.5) * (AR(SL_AREA + 1, 0) + AR(SL_AREA + 1, -di));
+                const T ihx = PR::div(L, tmax(Ae, eps));
+                const T mux = Cwh * be * ihx * ihx;
+                const T Ax = T(0.5) * (AR(SL_AREA + 0, 0) + AR(SL_AREA + 0, -dj));
+                const T ihe = PR::div(L, tmax(Ax, eps));
+                const T mue = Cwh * be * ihe * ihe;
+                val = Ecen + T(0.5) * mux * dB1i - T(0.5) * mue * dB0j;
+            }
+            hall[a] = st<MIX>(F, G, SL_TAPER + a, q) * val;
         }
 #undef AR
-        const T eh = st<MIX>(F, G, SL_TAPER + a, q) * val;
-        F[SL_EH + a][q] = (double)eh;
-        if (with_hall == 2) {
-            F[SL_E + a][q] = (double)E;
-            continue;
+    }
+    if (with_hall == 1) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            E[a] = E[a] + hall[a];
+            for (int f = 0; f < 6; ++f) {
+                const int nax = f >> 1;
+                if (bk.bc[f] != MBC_WALL || nax == a) continue;
+                if ((f & 1) ? (idx[nax] == bk.m[nax]) : (idx[nax] == 0)) E[a] = T(0);
+            }
         }
-        T e = E + eh;
-        for (int f = 0; f < 6; ++f) {
-            const int nax = f >> 1;
-            if (bk.bc[f] != MBC_WALL || nax == a) continue;
-            if ((f & 1) ? (idx[nax] == bk.m[nax]) : (idx[nax] == 0)) e = T(0);
-        }
-        F[SL_E + a][q] = (double)e;
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        if (idx[a] >= bk.m[a]) continue;
+        F[SL_E + a][q] = (double)E[a];
+        if (with_hall) F[SL_EH + a][q] = (double)hall[a];
     }
 #undef FB
 #undef FE
@@ -880,9 +919,13 @@ __global__ void k_edge_total(const MercRange R, const MercBlk *__restrict__ B, d
 
 // ---------------------------------------------------------------------------
 // (the RHS comes from the FP32 table in the mixed form; the accumulation is FP64)
-template <bool MIX>
+// The slots may alias for all the compiler knows, so it keeps every load behind
+// the stores before it: all loads of a point come first.  The box has at least
+// two ghost layers, so the edges one above a point can be read at every point
+// of the node range.
+template <bool MIX, int NS>
 __global__ void k_update_all(const MercRange R, const MercBlk *__restrict__ B, double *const *__restrict__ F_,
-                             const float *const *__restrict__ G_, const double *__restrict__ dtp, int ns) {
+                             const float *const *__restrict__ G_, const double *__restrict__ dtp) {
     gdouble *const *__restrict__ F = gslots(F_);
     const gfloat *const *__restrict__ G = gslots(G_);
     LOCATE(R);
@@ -890,33 +933,49 @@ __global__ void k_update_all(const MercRange R, const MercBlk *__restrict__ B, d
     const long long q = p.q, di = OI(p), dj = OJ(p), dk = 1;
     const double dt = dtp[bk.run];
     if (dt == 0.0) return;  // the run is stopped (k_dt_commit)
-    if (p.i < bk.m[0] && p.j < bk.m[1] && p.k < bk.m[2])
-        for (int m = 0; m < 5; ++m) {
-            // the fluid RHS is read here only, RHS_B written here and only downloaded:
-            // non-temporal, so they do not displace reused data from the caches
+    const bool ci = p.i < bk.m[0], cj = p.j < bk.m[1], ck = p.k < bk.m[2];
+    const bool cell = ci && cj && ck;
+    double u[NS][5];
+    const double e0 = F[SL_E + 0][q], e0k = F[SL_E + 0][q + dk], e0j = F[SL_E + 0][q + dj];
+    const double e1 = F[SL_E + 1][q], e1k = F[SL_E + 1][q + dk], e1i = F[SL_E + 1][q + di];
+    const double e2 = F[SL_E + 2][q], e2j = F[SL_E + 2][q + dj], e2i = F[SL_E + 2][q + di];
+    const double b0 = F[SL_B + 0][q], b1 = F[SL_B + 1][q], b2 = F[SL_B + 2][q];
+    if (cell) {
+        // the fluid RHS is read here only, RHS_B written here and only downloaded:
+        // non-temporal, so they do not displace reused data from the caches
+        double r[NS][5];
 #pragma unroll
-            for (int s = 0; s < MERC_NSMAX && s < ns; ++s) {
-                if constexpr (MIX) F[SPEC_U(s) + m][q] += dt * (double)__builtin_nontemporal_load(&G[SPEC_R(s) + m][q]);
-                else F[SPEC_U(s) + m][q] += dt * __builtin_nontemporal_load(&F[SPEC_R(s) + m][q]);
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int m = 0; m < 5; ++m) {
+                u[s][m] = F[SPEC_U(s) + m][q];
+                if constexpr (MIX) r[s][m] = (double)__builtin_nontemporal_load(&G[SPEC_R(s) + m][q]);
+                else r[s][m] = __builtin_nontemporal_load(&F[SPEC_R(s) + m][q]);
             }
-        }
-    if (p.j < bk.m[1] && p.k < bk.m[2]) {
-        const double c = (F[SL_E + 1][q] - F[SL_E + 1][q + dk]) + (F[SL_E + 2][q + dj] - F[SL_E + 2][q]);
-        const double r = -1.0 * c;
-        __builtin_nontemporal_store(r, &F[SL_RHSB + 0][q]);
-        F[SL_B + 0][q] += dt * r;
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int m = 0; m < 5; ++m) u[s][m] += dt * r[s][m];
     }
-    if (p.i < bk.m[0] && p.k < bk.m[2]) {
-        const double c = (F[SL_E + 0][q + dk] - F[SL_E + 0][q]) + (F[SL_E + 2][q] - F[SL_E + 2][q + di]);
-        const double r = -1.0 * c;
-        __builtin_nontemporal_store(r, &F[SL_RHSB + 1][q]);
-        F[SL_B + 1][q] += dt * r;
+    const double r0 = -1.0 * ((e1 - e1k) + (e2j - e2));
+    const double r1 = -1.0 * ((e0k - e0) + (e2 - e2i));
+    const double r2 = -1.0 * ((e0 - e0j) + (e1i - e1));
+    if (cell)
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int m = 0; m < 5; ++m) F[SPEC_U(s) + m][q] = u[s][m];
+    if (cj && ck) {
+        __builtin_nontemporal_store(r0, &F[SL_RHSB + 0][q]);
+        F[SL_B + 0][q] = b0 + dt * r0;
     }
-    if (p.i < bk.m[0] && p.j < bk.m[1]) {
-        const double c = (F[SL_E + 0][q] - F[SL_E + 0][q + dj]) + (F[SL_E + 1][q + di] - F[SL_E + 1][q]);
-        const double r = -1.0 * c;
-        __builtin_nontemporal_store(r, &F[SL_RHSB + 2][q]);
-        F[SL_B + 2][q] += dt * r;
+    if (ci && ck) {
+        __builtin_nontemporal_store(r1, &F[SL_RHSB + 1][q]);
+        F[SL_B + 1][q] = b1 + dt * r1;
+    }
+    if (ci && cj) {
+        __builtin_nontemporal_store(r2, &F[SL_RHSB + 2][q]);
+        F[SL_B + 2][q] = b2 + dt * r2;
     }
 }
 
@@ -926,21 +985,29 @@ DEVI void bcell_jedge_point(gdouble *const *__restrict__ F, const gfloat *const 
                             bool monitor, double &dmx, double &bmx) {
     using T = typename Prec<MIX>::T;
     const long long q = p.q, di = OI(p), dj = OJ(p), dk = 1;
-    if (p.i < bk.m[0] && p.j < bk.m[1] && p.k < bk.m[2]) {
-        T pt[6], pi[6];
-        pt[0] = -(T)F[SL_B + 0][q] - (T)F[SL_BADD + 0][q];
-        pt[1] = (T)F[SL_B + 0][q + di] + (T)F[SL_BADD + 0][q + di];
-        pt[2] = -(T)F[SL_B + 1][q] - (T)F[SL_BADD + 1][q];
-        pt[3] = (T)F[SL_B + 1][q + dj] + (T)F[SL_BADD + 1][q + dj];
-        pt[4] = -(T)F[SL_B + 2][q] - (T)F[SL_BADD + 2][q];
-        pt[5] = (T)F[SL_B + 2][q + 1] + (T)F[SL_BADD + 2][q + 1];
-        pi[0] = -(T)F[SL_B + 0][q];
-        pi[1] = (T)F[SL_B + 0][q + di];
-        pi[2] = -(T)F[SL_B + 1][q];
-        pi[3] = (T)F[SL_B + 1][q + dj];
-        pi[4] = -(T)F[SL_B + 2][q];
-        pi[5] = (T)F[SL_B + 2][q + 1];
-        T bt[3] = {T(0), T(0), T(0)}, bi[3] = {T(0), T(0), T(0)};
+    const bool ci = p.i < bk.m[0], cj = p.j < bk.m[1], ck = p.k < bk.m[2];
+    const bool cell = ci && cj && ck;
+    // every load of the point before its first store: the slots may alias for
+    // all the compiler knows, and it would load B and the weights again behind
+    // each store
+    const double b0 = F[SL_B + 0][q], b1 = F[SL_B + 1][q], b2 = F[SL_B + 2][q];
+    const double b0i = F[SL_B + 0][q + di], b1j = F[SL_B + 1][q + dj], b2k = F[SL_B + 2][q + dk];
+#define BB(a, o) (st<MIX>(F, G, SL_BETA + (a), q + (o)) * (T)F[SL_B + (a)][q + (o)])
+    const T h0 = st<MIX>(F, G, SL_BETA + 0, q) * (T)b0, h1 = st<MIX>(F, G, SL_BETA + 1, q) * (T)b1, h2 = st<MIX>(F, G, SL_BETA + 2, q) * (T)b2;
+    const T j0 = (T(1) * ((BB(1, -dk) - h1) + (h2 - BB(2, -dj)))) * st<MIX>(F, G, SL_ALPHA + 0, q);
+    const T j1 = (T(1) * ((h0 - BB(0, -dk)) + (BB(2, -di) - h2))) * st<MIX>(F, G, SL_ALPHA + 1, q);
+    const T j2 = (T(1) * ((BB(0, -dj) - h0) + (h1 - BB(1, -di)))) * st<MIX>(F, G, SL_ALPHA + 2, q);
+#undef BB
+    T bt[3] = {T(0), T(0), T(0)}, bi[3] = {T(0), T(0), T(0)};
+    if (cell) {
+        const T pi[6] = {-(T)b0, (T)b0i, -(T)b1, (T)b1j, -(T)b2, (T)b2k};
+        T pt[6];
+        pt[0] = -(T)b0 - (T)F[SL_BADD + 0][q];
+        pt[1] = (T)b0i + (T)F[SL_BADD + 0][q + di];
+        pt[2] = -(T)b1 - (T)F[SL_BADD + 1][q];
+        pt[3] = (T)b1j + (T)F[SL_BADD + 1][q + dj];
+        pt[4] = -(T)b2 - (T)F[SL_BADD + 2][q];
+        pt[5] = (T)b2k + (T)F[SL_BADD + 2][q + 1];
 #pragma unroll
         for (int n = 0; n < 6; ++n)
 #pragma unroll
@@ -949,35 +1016,22 @@ DEVI void bcell_jedge_point(gdouble *const *__restrict__ F, const gfloat *const 
                 bt[c] += w * pt[n];
                 bi[c] += w * pi[n];
             }
+    }
+    if (cell)
         for (int c = 0; c < 3; ++c) {
             F[SL_BC + c][q] = (double)bt[c];
             F[SL_BI + c][q] = (double)bi[c];
         }
-        if (monitor) {
-            // calc_divB's d2 B (the expression and order of k_divb)
-            const double d = (F[SL_B][q + di] - F[SL_B][q] + F[SL_B + 1][q + dj] - F[SL_B + 1][q] + F[SL_B + 2][q + 1] - F[SL_B + 2][q]);
-            dmx = dmax(dmx, fabs(d));
-        }
-    }
+    if (ci) F[SL_J + 0][q] = (double)j0;
+    if (cj) F[SL_J + 1][q] = (double)j1;
+    if (ck) F[SL_J + 2][q] = (double)j2;
     if (monitor) {
-        if (p.j < bk.m[1] && p.k < bk.m[2]) bmx = dmax(bmx, fabs(F[SL_B][q]));
-        if (p.i < bk.m[0] && p.k < bk.m[2]) bmx = dmax(bmx, fabs(F[SL_B + 1][q]));
-        if (p.i < bk.m[0] && p.j < bk.m[1]) bmx = dmax(bmx, fabs(F[SL_B + 2][q]));
+        // calc_divB's d2 B (the expression and order of k_divb)
+        if (cell) dmx = dmax(dmx, fabs(b0i - b0 + b1j - b1 + b2k - b2));
+        if (cj && ck) bmx = dmax(bmx, fabs(b0));
+        if (ci && ck) bmx = dmax(bmx, fabs(b1));
+        if (ci && cj) bmx = dmax(bmx, fabs(b2));
     }
-#define BB(a, o) (st<MIX>(F, G, SL_BETA + (a), q + (o)) * (T)F[SL_B + (a)][q + (o)])
-    if (p.i < bk.m[0]) {
-        const T v = (BB(1, -dk) - BB(1, 0)) + (BB(2, 0) - BB(2, -dj));
-        F[SL_J + 0][q] = (double)((T(1) * v) * st<MIX>(F, G, SL_ALPHA + 0, q));
-    }
-    if (p.j < bk.m[1]) {
-        const T v = (BB(0, 0) - BB(0, -dk)) + (BB(2, -di) - BB(2, 0));
-        F[SL_J + 1][q] = (double)((T(1) * v) * st<MIX>(F, G, SL_ALPHA + 1, q));
-    }
-    if (p.k < bk.m[2]) {
-        const T v = (BB(0, -dj) - BB(0, 0)) + (BB(1, 0) - BB(1, -di));
-        F[SL_J + 2][q] = (double)((T(1) * v) * st<MIX>(F, G, SL_ALPHA + 2, q));
-    }
-#undef BB
 }
 
 // max of two values over the workgroup, written to part[2 * blockIdx.x .. + 1]
@@ -1189,8 +1243,13 @@ void launch_edge_total(hipStream_t st, const RangeH &R, const MercBlk *B, double
 }
 void launch_update_all(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, const double *dt,
                        bool mix, int ns) {
-    if (mix) LAUNCH_R(k_update_all<true>, R, B, F, G, dt, ns);
-    else LAUNCH_R(k_update_all<false>, R, B, F, G, dt, ns);
+    if (mix) {
+        if (ns > 2) LAUNCH_R((k_update_all<true, 3>), R, B, F, G, dt);
+        else LAUNCH_R((k_update_all<true, 2>), R, B, F, G, dt);
+    } else {
+        if (ns > 2) LAUNCH_R((k_update_all<false, 3>), R, B, F, G, dt);
+        else LAUNCH_R((k_update_all<false, 2>), R, B, F, G, dt);
+    }
 }
 void launch_to_double(hipStream_t st, const float *src, double *dst, long long n) {
     if (n > 0) hipLaunchKernelGGL(k_to_double, dim3(nblk(n, 256)), dim3(256), 0, st, src, dst, n);
