@@ -113,6 +113,14 @@ struct MercRange {
 // sync plan and alias classes; the context adds no handler and no neighbour there
 enum MercBC { MBC_PERIODIC = 0, MBC_FARFIELD = 1, MBC_WALL = 2, MBC_INTERFACE = 3, MBC_EXTERNAL = 4 };
 
+// The time-step candidates of a run meet in DT_WORDS words, one of each 128-byte
+// line, and the smallest of them is the run's dt: workgroup b uses word b %
+// DT_WORDS.  Atomics on one word go one after another, about 18 ns each, and on a
+// small block every workgroup sends its own at the same moment.
+#define DT_WORDS 64
+#define DT_LINE 16  // words between two of them
+#define DT_RUN (DT_WORDS * DT_LINE)
+
 // slot sets of a merged sync op (passed by value as a kernel argument)
 #define MERC_MAX_SETS 12
 struct MultiSets {

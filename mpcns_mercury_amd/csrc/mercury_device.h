@@ -66,7 +66,12 @@ typedef __attribute__((address_space(1))) float gfloat;
 DEVI gdouble *const *gslots(double *const *F) { return static_cast<gdouble *const *>(static_cast<const void *>(F)); }
 DEVI const gfloat *const *gslots(const float *const *G) { return static_cast<const gfloat *const *>(static_cast<const void *>(G)); }
 
-// Minimum of the threads' time-step candidates per run, folded into dt_bits[run]
+// the word of a run that this workgroup's candidates go to
+DEVI unsigned long long *dt_word(unsigned long long *dt_bits, int run) {
+    return dt_bits + (long long)run * DT_RUN + (blockIdx.x % DT_WORDS) * DT_LINE;
+}
+
+// Minimum of the threads' time-step candidates per run, folded into the run's words
 // (FP64 bits, atomicMin: positive doubles order like their bit patterns).  A
 // workgroup whose located threads all belong to one run issues one atomic;
 // otherwise (a workgroup across a block boundary between runs) each wave whose
@@ -85,7 +90,7 @@ DEVI void dt_min_runs(double best, int run, unsigned long long *__restrict__ dt_
     }
     const bool wave_uniform = rmax < 0 || rmin == rmax;
     if (!wave_uniform) {
-        if (run >= 0 && best < 1e100) atomicMin(dt_bits + run, (unsigned long long)__double_as_longlong(best));
+        if (run >= 0 && best < 1e100) atomicMin(dt_word(dt_bits, run), (unsigned long long)__double_as_longlong(best));
         best = 1e100;
     }
     for (int off = 32; off > 0; off >>= 1) best = dmin(best, __shfl_xor(best, off, 64));
@@ -106,13 +111,25 @@ DEVI void dt_min_runs(double best, int run, unsigned long long *__restrict__ dt_
             if (r0 >= 0) {
                 double m = wmin[0];
                 for (int w = 1; w < nw; ++w) m = dmin(m, wmin[w]);
-                atomicMin(dt_bits + r0, (unsigned long long)__double_as_longlong(m));
+                atomicMin(dt_word(dt_bits, r0), (unsigned long long)__double_as_longlong(m));
             }
         } else {
             for (int w = 0; w < nw; ++w)
-                if (wrun[w] >= 0) atomicMin(dt_bits + wrun[w], (unsigned long long)__double_as_longlong(wmin[w]));
+                if (wrun[w] >= 0) atomicMin(dt_word(dt_bits, wrun[w]), (unsigned long long)__double_as_longlong(wmin[w]));
         }
     }
+}
+
+// the smallest of a run's dt words, by the 64 lanes of one wave (positive
+// doubles order like their bit patterns)
+DEVI unsigned long long dt_fold(const unsigned long long *__restrict__ dt_bits, int run) {
+    static_assert(DT_WORDS == 64, "one word per lane");
+    unsigned long long v = dt_bits[(long long)run * DT_RUN + (threadIdx.x & 63) * DT_LINE];
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long o = __shfl_xor(v, off, 64);
+        v = o < v ? o : v;
+    }
+    return v;
 }
 
 // neighbour offsets

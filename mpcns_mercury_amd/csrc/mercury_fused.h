@@ -11,7 +11,7 @@ void launch_rhs_cell(hipStream_t st, const RangeH &R, const MercBlk *B, double *
 // each, marching over C planes along i (the LDS-tiled flux pass)
 void launch_rhs_tile(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, const MercPhys &P,
                      int C, bool mix);
-// dt_next: one word per run (nruns of them), reduced per run
+// dt_next: DT_RUN words per run (nruns of them), which hold no candidate yet (launch_dt_init, or launch_jcell_t)
 void launch_cell_end(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, const MercPhys &P,
                      unsigned long long *dt_next, int compute_dt, bool mix, int nruns);
 // ambi: also the node electron pressure of the ambipolar EMF (read by k_edge_total)
@@ -28,8 +28,10 @@ void launch_to_double(hipStream_t st, const float *src, double *dst, long long n
 void launch_bcell_jedge(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, bool mix,
                         double *divb_part = nullptr, double *divb_mon = nullptr);
 void launch_divb_monitor_reset(hipStream_t st, double *divb_mon);
-void launch_jcell_t(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, bool mix);
+// dt_next, when not null: also clears the dt words of the nruns runs
+void launch_jcell_t(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, bool mix,
+                    unsigned long long *dt_next = nullptr, int nruns = 0);
 void launch_to_float(hipStream_t st, const double *src, float *dst, long long n);
-// per run: the abort rule on dt_next[r], dt[r] committed, status 4 words per run
+// per run: the abort rule on the smallest of its dt words, dt[r] committed, status 4 words per run
 void launch_dt_commit(hipStream_t st, unsigned long long *dt, const unsigned long long *dt_next, unsigned long long *status, int nruns);
 }  // namespace merc

@@ -1122,10 +1122,15 @@ __global__ void k_bcell_jedge(const MercRange R, const MercBlk *__restrict__ B, 
     if (divb_part) group_max2(dmx, bmx, divb_part);
 }
 
-// calc_Jcell (MercurySolver_Current.cpp:203-259), owned cells
+// calc_Jcell (MercurySolver_Current.cpp:203-259), owned cells.  With dt_next it
+// also clears the nwords dt words that the derived pass behind it fills (a launch
+// of their own costs a small step more than the clearing does).
 template <bool MIX>
 __global__ void k_jcell_t(const MercRange R, const MercBlk *__restrict__ B, double *const *__restrict__ F_,
-                          const float *const *__restrict__ G_) {
+                          const float *const *__restrict__ G_, unsigned long long *__restrict__ dt_next, int nwords) {
+    if (dt_next)
+        for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nwords; t += gridDim.x * blockDim.x)
+            dt_next[(long long)t * DT_LINE] = (unsigned long long)__double_as_longlong(1e100);
     gdouble *const *__restrict__ F = gslots(F_);
     const gfloat *const *__restrict__ G = gslots(G_);
     using T = typename Prec<MIX>::T;
@@ -1160,12 +1165,12 @@ __global__ void k_to_float(const double *__restrict__ src, float *__restrict__ d
 // passes skip their writes when dt is 0 (no valid step has dt = 0), so the
 // state stays that of the last completed step, as the reference exits before
 // its update.
-// One thread per run of the context (status: 4 words per run).
-__global__ void k_dt_commit(unsigned long long *dt, const unsigned long long *dt_next, unsigned long long *status, int nruns) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= nruns) return;
+// One wave per run of the context (status: 4 words per run).
+__global__ void __launch_bounds__(64) k_dt_commit(unsigned long long *dt, const unsigned long long *dt_next, unsigned long long *status) {
+    const int r = blockIdx.x;
+    const unsigned long long bits = dt_fold(dt_next, r);
+    if (threadIdx.x != 0) return;
     unsigned long long *st = status + 4 * r;
-    const unsigned long long bits = dt_next[r];
     const double d = __longlong_as_double((long long)bits);
     if (st[0] != 0ULL) {
         dt[r] = 0ULL;
@@ -1177,10 +1182,6 @@ __global__ void k_dt_commit(unsigned long long *dt, const unsigned long long *dt
         dt[r] = bits;
         st[1] += 1ULL;
     }
-}
-__global__ void k_dt_reset(unsigned long long *dt_next, int nruns) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nruns) dt_next[r] = (unsigned long long)__double_as_longlong(1e100);
 }
 
 }  // namespace
@@ -1219,7 +1220,6 @@ void launch_rhs_tile(hipStream_t st, const RangeH &R, const MercBlk *B, double *
 }
 void launch_cell_end(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, const MercPhys &P,
                      unsigned long long *dt_next, int compute_dt, bool mix, int nruns) {
-    if (compute_dt) hipLaunchKernelGGL(k_dt_reset, dim3(nblk(nruns, 64)), dim3(64), 0, st, dt_next, nruns);
     const bool three = P.n_species >= 3.0, ens = nruns > 1;
 #define CELL_END(M, N, E) LAUNCH_R((k_cell_end<M, N, E>), R, B, F, G, P, dt_next, compute_dt)
     if (mix) {
@@ -1264,15 +1264,16 @@ void launch_bcell_jedge(hipStream_t st, const RangeH &R, const MercBlk *B, doubl
 void launch_divb_monitor_reset(hipStream_t st, double *divb_mon) {
     hipLaunchKernelGGL(k_divb_monitor_reset, dim3(1), dim3(64), 0, st, divb_mon);
 }
-void launch_jcell_t(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, bool mix) {
-    if (mix) LAUNCH_R(k_jcell_t<true>, R, B, F, G);
-    else LAUNCH_R(k_jcell_t<false>, R, B, F, G);
+void launch_jcell_t(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, bool mix,
+                    unsigned long long *dt_next, int nruns) {
+    if (mix) LAUNCH_R(k_jcell_t<true>, R, B, F, G, dt_next, nruns * DT_WORDS);
+    else LAUNCH_R(k_jcell_t<false>, R, B, F, G, dt_next, nruns * DT_WORDS);
 }
 void launch_to_float(hipStream_t st, const double *src, float *dst, long long n) {
     if (n > 0) hipLaunchKernelGGL(k_to_float, dim3(nblk(n, 256)), dim3(256), 0, st, src, dst, n);
 }
 void launch_dt_commit(hipStream_t st, unsigned long long *dt, const unsigned long long *dt_next, unsigned long long *status, int nruns) {
-    hipLaunchKernelGGL(k_dt_commit, dim3(nblk(nruns, 64)), dim3(64), 0, st, dt, dt_next, status, nruns);
+    hipLaunchKernelGGL(k_dt_commit, dim3(nruns), dim3(64), 0, st, dt, dt_next, status);
 }
 
 }  // namespace merc

@@ -738,7 +738,8 @@ public:
     hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_fork2 = nullptr, ev_join2 = nullptr;
     bool overlap = true;
     unsigned long long *d_dt = nullptr;       // dt word (double bits)
-    unsigned long long *d_dt_next = nullptr;  // next step's dt, reduced at the end of the derived fields
+    unsigned long long *d_dt_next = nullptr;  // next step's dt words (DT_RUN per run), filled at the end of the derived fields
+    unsigned long long *d_dt_now = nullptr;   // the same of mercury_timestep, which leaves the pending ones alone
     // run status written by k_dt_commit: [0] stop code (1 = dt underflow, sticky),
     // [1] steps committed since the status was cleared, [2] bits of the refused dt
     unsigned long long *d_status = nullptr;
@@ -865,7 +866,9 @@ public:
         }
         F->upload_blocks();
         HIPCHK(hipMalloc(&d_dt, sizeof(unsigned long long) * nruns));
-        HIPCHK(hipMalloc(&d_dt_next, sizeof(unsigned long long) * nruns));
+        HIPCHK(hipMalloc(&d_dt_next, sizeof(unsigned long long) * DT_RUN * nruns));
+        HIPCHK(hipMalloc(&d_dt_now, sizeof(unsigned long long) * DT_RUN * nruns));
+        HIPCHK(hipMemset(d_dt_next, 0, sizeof(unsigned long long) * DT_RUN * nruns));
         HIPCHK(hipMalloc(&d_status, 4 * sizeof(unsigned long long) * nruns));
         HIPCHK(hipMemset(d_status, 0, 4 * sizeof(unsigned long long) * nruns));
         HIPCHK(hipMalloc(&d_red, 2 * sizeof(unsigned long long)));
@@ -949,6 +952,7 @@ public:
         if (graph) (void)hipGraphDestroy(graph);
         if (d_dt) (void)hipFree(d_dt);
         if (d_dt_next) (void)hipFree(d_dt_next);
+        if (d_dt_now) (void)hipFree(d_dt_now);
         if (d_status) (void)hipFree(d_status);
         if (farena) (void)hipFree(farena);
         if (fptr) (void)hipFree(fptr);
@@ -1678,7 +1682,7 @@ public:
         alias.launch(st, Fd(), SL_J);
         singular_current(SL_B, SL_J);
         run_merged(MG_DERIVED_PAIR);
-        launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix());
+        launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix(), final ? d_dt_next : nullptr, nruns);
         sync(G_JCELL);
         launch_cell_end(st, R_box.h, Bd(), Fd(), Gd(), P, d_dt_next, final ? 1 : 0, mix(), nruns);
     }
@@ -1710,7 +1714,7 @@ public:
         } else {
             run_merged(MG_DERIVED_PAIR, st);
         }
-        launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix());
+        launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix(), final ? d_dt_next : nullptr, nruns);
         sync(G_JCELL);
         HIPCHK(hipEventRecord(ev_join2, st2));
         HIPCHK(hipStreamWaitEvent(st, ev_join2, 0));
@@ -1978,6 +1982,7 @@ public:
         } else {
             derived();
             refresh_float_statics();
+            launch_dt_init(st, d_dt_next, nruns);
             launch_cell_end(st, R_box.h, Bd(), Fd(), Gd(), P, d_dt_next, 1, false, nruns);
         }
         prepared = true;
@@ -2028,10 +2033,16 @@ public:
             singular_current(SL_B, SL_J);
         else if (op == "alias_j")
             alias.launch(st, Fd(), SL_J);
-        else if (op == "timestep") launch_timestep(st, R_cell.h, Bd(), Fd(), P, d_dt, nruns);
+        else if (op == "timestep") {
+            launch_timestep(st, R_cell.h, Bd(), Fd(), P, d_dt_now, nruns);
+            launch_dt_fold(st, d_dt, d_dt_now, nruns);
+        }
         else if (op == "stage") stage();
         else if (op == "rhs_cell") launch_flux(st);
-        else if (op == "cell_end") launch_cell_end(st, R_box.h, Bd(), Fd(), Gd(), P, d_dt_next, 1, mix(), nruns);
+        else if (op == "cell_end") {
+            launch_dt_init(st, d_dt_next, nruns);
+            launch_cell_end(st, R_box.h, Bd(), Fd(), Gd(), P, d_dt_next, 1, mix(), nruns);
+        }
         else if (op == "eface_u") launch_eface_u(st, R_eface.h, Bd(), Fd(), Gd(), mix(), P.ambipolar_enabled != 0.0, nspecies());
         else if (op == "edge_total") launch_edge_total(st, R_node.h, Bd(), Fd(), Gd(), P, alias.n == 0 ? 1 : 0, mix());
         else if (op == "update_all") launch_update_all(st, R_node.h, Bd(), Fd(), Gd(), dtp(), mix(), nspecies());

@@ -16,9 +16,11 @@ void launch_pv_uplus(hipStream_t st, const RangeH &R, const MercBlk *B, double *
 void launch_bcell(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F);
 void launch_jedge(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, int s_face = SL_B, int s_edge = SL_J);
 void launch_jcell(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F);
-// dt_bits: one word per run (nruns of them), each the minimum over its run's cells
+// dt_bits: DT_RUN words per run; the smallest of a run's is the minimum over its cells
 void launch_timestep(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const MercPhys &P, unsigned long long *dt_bits,
                      int nruns);
+void launch_dt_init(hipStream_t st, unsigned long long *dt_bits, int nruns);
+void launch_dt_fold(hipStream_t st, unsigned long long *dt, const unsigned long long *dt_bits, int nruns);
 void launch_flux_div(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const MercPhys &P);
 void launch_sources(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const MercPhys &P);
 void launch_eface(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F);

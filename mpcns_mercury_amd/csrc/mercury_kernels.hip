@@ -576,21 +576,31 @@ __global__ void k_rk2(const MercRange R, const MercBlk *__restrict__ B, double *
     const long long q = p.q;
     const bool cell = p.i < bk.m[0] && p.j < bk.m[1] && p.k < bk.m[2];
     const bool face[3] = {p.j < bk.m[1] && p.k < bk.m[2], p.i < bk.m[0] && p.k < bk.m[2], p.i < bk.m[0] && p.j < bk.m[1]};
-    if (save) {
-        if (cell)
-            for (int m = 0; m < 5; ++m)
+    // every read of the point before its first write (the slots may alias for
+    // the compiler): one memory latency in place of thirteen
+    double u[MERC_NSMAX][5], b[3];
 #pragma unroll
-                for (int s = 0; s < MERC_NSMAX && s < ns; ++s) F[SPEC_U0(s) + m][q] = F[SPEC_U(s) + m][q];
-        for (int a = 0; a < 3; ++a)
-            if (face[a]) F[SL_B0 + a][q] = F[SL_B + a][q];
-    } else {
-        if (cell)
-            for (int m = 0; m < 5; ++m)
+    for (int s = 0; s < MERC_NSMAX; ++s)
+        if (cell && s < ns)
 #pragma unroll
-                for (int s = 0; s < MERC_NSMAX && s < ns; ++s) F[SPEC_U(s) + m][q] = 0.5 * (F[SPEC_U0(s) + m][q] + F[SPEC_U(s) + m][q]);
-        for (int a = 0; a < 3; ++a)
-            if (face[a]) F[SL_B + a][q] = 0.5 * (F[SL_B0 + a][q] + F[SL_B + a][q]);
-    }
+            for (int m = 0; m < 5; ++m) {
+                u[s][m] = F[SPEC_U(s) + m][q];
+                if (!save) u[s][m] = 0.5 * (F[SPEC_U0(s) + m][q] + u[s][m]);
+            }
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        if (face[a]) {
+            b[a] = F[SL_B + a][q];
+            if (!save) b[a] = 0.5 * (F[SL_B0 + a][q] + b[a]);
+        }
+#pragma unroll
+    for (int s = 0; s < MERC_NSMAX; ++s)
+        if (cell && s < ns)
+#pragma unroll
+            for (int m = 0; m < 5; ++m) F[(save ? SPEC_U0(s) : SPEC_U(s)) + m][q] = u[s][m];
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        if (face[a]) F[(save ? SL_B0 : SL_B) + a][q] = b[a];
 }
 
 // ---------------------------------------------------------------------------
@@ -838,10 +848,15 @@ __global__ void k_zero_span(double *const *__restrict__ F_, const SlotSet S, lon
     for (int c = 0; c < S.n; ++c) F[S.s[c]][t] = 0.0;
 }
 
-// dt word initialisation inside the step
+// the dt words of every run without a candidate
 __global__ void k_dt_init(unsigned long long *dt_bits, int nruns) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < nruns) dt_bits[r] = (unsigned long long)__double_as_longlong(1e100);
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < nruns * DT_WORDS) dt_bits[(long long)t * DT_LINE] = (unsigned long long)__double_as_longlong(1e100);
+}
+// dt[r] <- the smallest of run r's words (one wave per run)
+__global__ void __launch_bounds__(64) k_dt_fold(unsigned long long *dt, const unsigned long long *dt_bits) {
+    const unsigned long long v = dt_fold(dt_bits, blockIdx.x);
+    if (threadIdx.x == 0) dt[blockIdx.x] = v;
 }
 
 }  // namespace
@@ -863,8 +878,14 @@ void launch_jedge(hipStream_t st, const RangeH &R, const MercBlk *B, double *con
 void launch_jcell(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F) { LAUNCH_R(k_jcell, R, B, F); }
 void launch_timestep(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const MercPhys &P, unsigned long long *dt_bits,
                      int nruns) {
-    hipLaunchKernelGGL(k_dt_init, dim3(nblk(nruns, 64)), dim3(64), 0, st, dt_bits, nruns);
+    launch_dt_init(st, dt_bits, nruns);
     LAUNCH_R(k_timestep, R, B, F, P, dt_bits);
+}
+void launch_dt_init(hipStream_t st, unsigned long long *dt_bits, int nruns) {
+    hipLaunchKernelGGL(k_dt_init, dim3(nblk(nruns * DT_WORDS, 64)), dim3(64), 0, st, dt_bits, nruns);
+}
+void launch_dt_fold(hipStream_t st, unsigned long long *dt, const unsigned long long *dt_bits, int nruns) {
+    hipLaunchKernelGGL(k_dt_fold, dim3(nruns), dim3(64), 0, st, dt, dt_bits);
 }
 void launch_flux_div(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const MercPhys &P) { LAUNCH_R(k_flux_div, R, B, F, P); }
 void launch_sources(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const MercPhys &P) { LAUNCH_R(k_sources, R, B, F, P); }
