@@ -12,8 +12,6 @@
 #pragma once
 #include <stdint.h>
 
-#define MERC_MAX_SYNC_SLOTS 10
-
 // stagger locations (include/0_basic/StaggerLocation.h)
 enum MercLoc { LOC_CELL = 0, LOC_FX, LOC_FY, LOC_FZ, LOC_EX, LOC_EY, LOC_EZ, LOC_NODE };
 
@@ -121,10 +119,18 @@ enum MercBC { MBC_PERIODIC = 0, MBC_FARFIELD = 1, MBC_WALL = 2, MBC_INTERFACE = 
 #define DT_LINE 16  // words between two of them
 #define DT_RUN (DT_WORDS * DT_LINE)
 
-// slot sets of a merged sync op (passed by value as a kernel argument)
-#define MERC_MAX_SETS 12
-struct MultiSets {
-    int n[MERC_MAX_SETS];
-    int s[MERC_MAX_SETS][MERC_MAX_SYNC_SLOTS];
-    double v[MERC_MAX_SETS][MERC_MAX_SYNC_SLOTS];
+// One wave of a sync launch: 64 entries (dst, src) of one kind and one field.
+// COPY: every component of dst <- src.  CONST: component c of dst <- the value
+// table at src + c (a far-field state, a value of its own per entry).  WALL1 and
+// WALL2: the reflected state at a solid surface, once (the first layer) or twice
+// (the ghosts, made from the first layer) over the state at src, the cell behind
+// the first layer.  CHAIN: dst is an aliased value that goes to up to 2 np ghosts
+// before its owner's value, src, replaces it; the ghosts follow, two to an entry,
+// the n-th pair of a lane 64 n entries further.
+enum SyncKind { SYNC_COPY = 0, SYNC_CONST, SYNC_WALL1, SYNC_WALL2, SYNC_CHAIN };
+struct SyncWave {
+    int kind, slot, ncomp;
+    int first;    // first entry
+    int species;  // WALL1, WALL2: 0 H+, 2 He++
+    int np;       // CHAIN: pairs of ghosts
 };

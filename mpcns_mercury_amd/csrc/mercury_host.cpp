@@ -12,10 +12,13 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
+#include <climits>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <future>
 #include <initializer_list>
 #include <map>
 #include <memory>
@@ -291,7 +294,7 @@ static void make_range(const Field &F, int lo_off, int hi_off, RangeOwner &R) {
 // ---------------------------------------------------------------------------
 // synchronisation programs
 // ---------------------------------------------------------------------------
-enum OpType { OP_COPY, OP_FILL, OP_SETV, OP_WALLF, OP_ZERO };
+enum OpType { OP_COPY, OP_FILL, OP_SETV, OP_WALLF };
 
 // one operation of one field (or of fields sharing an index list) in one
 // phase of a group's program; host lists only
@@ -299,7 +302,7 @@ struct SyncOp {
     OpType type;
     int phase = 0;
     std::vector<int> slots;
-    std::vector<double> fillv;
+    std::vector<double> fillv;  // FILL: a value per slot; WALLF of Na+: the ghosts' state
     int is_na = 0;  // WALLF: species (0 H+, 1 Na+, 2 He++)
     std::vector<int> hidx;     // pairs for COPY, (first, deeper, ghosts) for WALLF
     std::vector<double> hval;  // SETV values
@@ -309,18 +312,207 @@ struct GroupProg {
     std::vector<std::unique_ptr<SyncOp>> ops;
 };
 
-// A merged launch: every op of one type in one phase of a set of independent
-// groups. Entries name their slot set: COPY (dst, src, set), FILL (dst, set),
-// SETV (dst, slot) + value, WALLF (slot, species, first, deeper, g ghosts).
-struct MergedOp {
-    OpType type;
-    MultiSets S{};
-    DBuf<int> ent;
-    DBuf<double> val;
-    long long n = 0;
+// The launches of a set of independent groups' syncs (SyncPlan), on the device:
+// per launch its waves, entries and values, in one buffer for the set.
+struct SyncLaunch {
+    const SyncWave *waves;
+    long long nw;
+    const int *ent;
+    const double *val;
 };
-struct MergedProg {
-    std::vector<std::unique_ptr<MergedOp>> ops;
+struct SyncProg {
+    DBuf<double> mem;
+    std::vector<SyncLaunch> launches;
+};
+
+// Turns the phases of a field's sync into as few launches as can be.  It follows
+// the ops in order, symbolically: what each value is after them, in terms of the
+// values before the first: a copy of one, a constant, or a wall state made of the
+// cell behind the wall's first layer.  A launch then writes every changed value
+// from there, whatever the number of phases (three to six launches of about 5 us
+// each before, one behind the other).
+//
+// Threads of a launch run in no order, so a value that others read must not be
+// written in the same launch.  The one exception is an aliased value, which ghosts
+// copy before its owner's value replaces it: one thread makes those copies and
+// then the replacement (a chain).  Where the ops cannot be joined under these
+// rules, the longest run of them that can makes a launch and the rest follow.
+class SyncPlan {
+public:
+    explicit SyncPlan(long long nvalues) : sym(nvalues, {NONE, 0}) {}
+    // appends one field's sync: ops in program order that touch slots slot ..
+    // slot + ncomp - 1; launch n of every field goes to the same kernel launch
+    void add(const std::vector<const SyncOp *> &ops, int slot, int ncomp, int g) {
+        // where a launch may end: not between the components of one set of values
+        std::vector<size_t> ends;
+        for (size_t n = 0; n < ops.size(); ++n) {
+            if (ops[n]->type == OP_SETV) n += ncomp - 1;
+            ends.push_back(n + 1);
+        }
+        size_t at = 0, launch = 0;
+        for (size_t u = 0; u < ends.size();) {
+            size_t last = ends.size() - 1;
+            // one op by itself always can: no destination of it is a source of it
+            while (!(follow(ops, at, ends[last], slot, ncomp, g) && joins()) && last > u) --last;
+            emit(launch++, slot, ncomp);
+            at = ends[last];
+            u = last + 1;
+        }
+    }
+    struct Host {
+        std::vector<SyncWave> waves;
+        std::vector<int> ent;
+        std::vector<double> val;
+        // appends the waves of another group's launch
+        void append(const Host &o) {
+            const int e0 = (int)(ent.size() / 2), v0 = (int)val.size();
+            ent.insert(ent.end(), o.ent.begin(), o.ent.end());
+            val.insert(val.end(), o.val.begin(), o.val.end());
+            for (SyncWave w : o.waves) {
+                w.first += e0;
+                if (w.kind == SYNC_CONST)
+                    for (int l = 0; l < 64; ++l) ent[2 * ((size_t)w.first + l) + 1] += v0;
+                waves.push_back(w);
+            }
+        }
+    };
+    std::vector<Host> out;
+
+private:
+    enum { NONE = 0, RAW, CST, WALL_FIRST, WALL_GHOST };
+    struct Sym {
+        int type, a;
+    };
+    std::vector<Sym> sym;  // per value index: what it is after the ops followed so far
+    std::vector<int> touched;
+    std::vector<double> rows;  // constants, ncomp each
+    int wall_species = 0;
+    std::vector<std::pair<int, int>> chain;  // (aliased value, a ghost that copies it)
+    static constexpr size_t kWaveEntries = 64;
+
+    void set(int d, Sym v) {
+        if (sym[d].type == NONE) touched.push_back(d);
+        sym[d] = v;
+    }
+    Sym value_of(int s) const { return sym[s].type == NONE ? Sym{RAW, s} : sym[s]; }
+    int row(const double *v, int ncomp) {
+        if (rows.size() < (size_t)ncomp || std::memcmp(rows.data() + rows.size() - ncomp, v, sizeof(double) * ncomp) != 0)
+            rows.insert(rows.end(), v, v + ncomp);
+        return (int)rows.size() - ncomp;
+    }
+    void reset() {
+        for (int d : touched) sym[d] = {NONE, 0};
+        touched.clear();
+        rows.clear();
+    }
+    // false: a wall op needs the value of a cell that an op before it changes
+    bool follow(const std::vector<const SyncOp *> &ops, size_t b, size_t e, int slot, int ncomp, int g) {
+        reset();
+        for (size_t n = b; n < e; ++n) {
+            const SyncOp &o = *ops[n];
+            const size_t c0 = std::find(o.slots.begin(), o.slots.end(), slot) - o.slots.begin();
+            if (o.type == OP_FILL) {
+                for (int d : o.hidx) set(d, {CST, row(o.fillv.data() + c0, ncomp)});
+            } else if (o.type == OP_SETV) {
+                // values of their own per entry, one op per component over the same entries
+                std::vector<double> v(ncomp);
+                for (size_t t = 0; t < o.hidx.size(); ++t) {
+                    for (int c = 0; c < ncomp; ++c) v[c] = ops[n + c]->hval[t];
+                    set(o.hidx[t], {CST, row(v.data(), ncomp)});
+                }
+                n += ncomp - 1;
+            } else if (o.type == OP_WALLF) {
+                wall_species = o.is_na;
+                for (size_t t = 0; t + 2 + g <= o.hidx.size(); t += 2 + g) {
+                    const int *w = &o.hidx[t];
+                    if (o.is_na == 1) {  // Na+: a floor state in the ghosts
+                        for (int l = 0; l < g; ++l) set(w[2 + l], {CST, row(o.fillv.data(), ncomp)});
+                        continue;
+                    }
+                    if (sym[w[1]].type != NONE) return false;
+                    set(w[0], {WALL_FIRST, w[1]});
+                    for (int l = 0; l < g; ++l) set(w[2 + l], {WALL_GHOST, w[1]});
+                }
+            } else {
+                for (size_t t = 0; t + 1 < o.hidx.size(); t += 2) set(o.hidx[t], value_of(o.hidx[t + 1]));
+            }
+        }
+        return true;
+    }
+    // whether the values can be written in one launch; collects the chains
+    bool joins() {
+        chain.clear();
+        for (int d : touched) {
+            const Sym v = sym[d];
+            if (v.type == CST || sym[v.a].type == NONE || (v.type == RAW && v.a == d)) continue;
+            if (v.type != RAW) return false;  // a wall state of a value that is written
+            chain.push_back({v.a, d});
+        }
+        std::sort(chain.begin(), chain.end());
+        auto read = [&](int x) {
+            const auto it = std::lower_bound(chain.begin(), chain.end(), std::make_pair(x, INT_MIN));
+            return it != chain.end() && it->first == x;
+        };
+        for (const auto &p : chain) {
+            const Sym v = sym[p.first];
+            // the value read is replaced by an unchanged one, and the reader is read by nobody
+            if (v.type != RAW || sym[v.a].type != NONE || read(p.second)) return false;
+        }
+        return true;
+    }
+    void emit(size_t launch, int slot, int ncomp) {
+        if (out.size() <= launch) out.resize(launch + 1);
+        Host &H = out[launch];
+        std::vector<int> part[SYNC_CHAIN];
+        const int base = (int)H.val.size();
+        H.val.insert(H.val.end(), rows.begin(), rows.end());
+        for (int d : touched) {
+            const Sym v = sym[d];
+            if (v.type == RAW) {
+                if (v.a == d || sym[v.a].type != NONE) continue;  // unchanged, or part of a chain
+                if (!chain.empty()) {
+                    const auto it = std::lower_bound(chain.begin(), chain.end(), std::make_pair(d, INT_MIN));
+                    if (it != chain.end() && it->first == d) continue;  // the end of a chain
+                }
+                part[SYNC_COPY].insert(part[SYNC_COPY].end(), {d, v.a});
+            } else if (v.type == CST) {
+                part[SYNC_CONST].insert(part[SYNC_CONST].end(), {d, base + v.a});
+            } else {
+                std::vector<int> &q = part[v.type == WALL_FIRST ? SYNC_WALL1 : SYNC_WALL2];
+                q.insert(q.end(), {d, v.a});
+            }
+        }
+        for (int kind = 0; kind < SYNC_CHAIN; ++kind)
+            for (size_t t = 0; t < part[kind].size(); t += 2 * kWaveEntries) {
+                H.waves.push_back(SyncWave{kind, slot, ncomp, (int)(H.ent.size() / 2), wall_species, 0});
+                const size_t n = std::min(2 * kWaveEntries, part[kind].size() - t);
+                H.ent.insert(H.ent.end(), part[kind].begin() + t, part[kind].begin() + t + n);
+                H.ent.resize(H.ent.size() + 2 * kWaveEntries - n, -1);
+            }
+        // chains, 64 a wave: (aliased value, owner), then the ghosts that read it
+        std::vector<std::pair<int, int>> lane;  // (number of ghosts, first in chain), the short ones first
+        for (size_t t = 0, u; t < chain.size(); t = u) {
+            for (u = t + 1; u < chain.size() && chain[u].first == chain[t].first;) ++u;
+            lane.push_back({(int)(u - t), (int)t});
+        }
+        std::sort(lane.begin(), lane.end());
+        for (size_t t = 0; t < lane.size(); t += kWaveEntries) {
+            const size_t n = std::min(kWaveEntries, lane.size() - t);
+            const int np = (lane[t + n - 1].first + 1) / 2;
+            H.waves.push_back(SyncWave{SYNC_CHAIN, slot, ncomp, (int)(H.ent.size() / 2), 0, np});
+            const size_t e0 = H.ent.size();
+            H.ent.resize(e0 + 2 * kWaveEntries * (1 + np), -1);
+            for (size_t l = 0; l < n; ++l) {
+                const auto &c = lane[t + l];
+                const int x = chain[c.second].first;
+                H.ent[e0 + 2 * l] = x;
+                H.ent[e0 + 2 * l + 1] = sym[x].a;
+                for (int u = 0; u < c.first; ++u) H.ent[e0 + 2 * (kWaveEntries * (1 + u / 2) + l) + u % 2] = chain[c.second + u].second;
+            }
+        }
+        reset();
+        chain.clear();
+    }
 };
 
 enum GroupId { G_UCELL = 0, G_BFACE, G_EEDGE, G_EHALL, G_JEDGE, G_BCELL, G_JCELL, G_BADD, G_ERES, G_ERES0, G_DB, G_NGROUP };
@@ -696,7 +888,7 @@ public:
     RangeOwner R_tile;   // tiled flux pass: ceil(m0 / tile_c) x ceil(m1 / 16) x ceil(m2 / 16) tiles per block
     int tile_c = 0;      // planes per tile along i; 0: the column kernel runs
     GroupProg prog[G_NGROUP];
-    std::map<unsigned, MergedProg> mprog;  // keyed by the bit set of groups
+    std::map<unsigned, SyncProg> mprog;  // keyed by the bit set of groups
     // caller sync plans: per group, stage 0 stands in for the context's own
     // halo copies and stage 1 for its owner -> alias copies; entries
     // (dst slot, dst, src slot, src, sign) on arena indices
@@ -866,8 +1058,8 @@ public:
         }
         F->upload_blocks();
         HIPCHK(hipMalloc(&d_dt, sizeof(unsigned long long) * nruns));
-        HIPCHK(hipMalloc(&d_dt_next, sizeof(unsigned long long) * DT_RUN * nruns));
-        HIPCHK(hipMalloc(&d_dt_now, sizeof(unsigned long long) * DT_RUN * nruns));
+        HIPCHK(hipMalloc(&d_dt_next, 2 * sizeof(unsigned long long) * DT_RUN * nruns));
+        d_dt_now = d_dt_next + DT_RUN * (size_t)nruns;
         HIPCHK(hipMemset(d_dt_next, 0, sizeof(unsigned long long) * DT_RUN * nruns));
         HIPCHK(hipMalloc(&d_status, 4 * sizeof(unsigned long long) * nruns));
         HIPCHK(hipMemset(d_status, 0, 4 * sizeof(unsigned long long) * nruns));
@@ -952,7 +1144,6 @@ public:
         if (graph) (void)hipGraphDestroy(graph);
         if (d_dt) (void)hipFree(d_dt);
         if (d_dt_next) (void)hipFree(d_dt_next);
-        if (d_dt_now) (void)hipFree(d_dt_now);
         if (d_status) (void)hipFree(d_status);
         if (farena) (void)hipFree(farena);
         if (fptr) (void)hipFree(fptr);
@@ -1068,7 +1259,7 @@ public:
                 if (idx.empty()) return;
                 if (t == OP_COPY)
                     for (auto &o : ph)
-                        if (o->type == OP_COPY && o->hidx == idx && o->slots.size() + slots.size() <= MERC_MAX_SYNC_SLOTS) {
+                        if (o->type == OP_COPY && o->hidx == idx) {
                             o->slots.insert(o->slots.end(), slots.begin(), slots.end());
                             return;
                         }
@@ -1180,7 +1371,9 @@ public:
                     if (!fill_d[c].empty()) add(A, OP_SETV, {sl[c]}, std::move(fill_d[c]), std::move(fill_v[c]));
                 if (!setd.empty()) add(A, OP_SETV, sl, std::move(setd), std::move(setv));
                 add(Bc, OP_COPY, sl, std::move(copyB));
-                if (!wallC.empty()) add(C, OP_WALLF, sl, std::move(wallC), {}, nullptr, gf.kind == K_UNA ? 1 : (gf.kind == K_UHE ? 2 : 0));
+                const double na_floor[5] = {P.wall_rho_floor_Na, 0.0, 0.0, 0.0, P.wall_p_floor / (P.gamma - 1.0)};
+                if (!wallC.empty())
+                    add(C, OP_WALLF, sl, std::move(wallC), {}, gf.kind == K_UNA ? na_floor : nullptr, gf.kind == K_UNA ? 1 : (gf.kind == K_UHE ? 2 : 0));
                 if (!zeroC.empty()) {
                     static const double z[10] = {0};
                     add(C, OP_FILL, sl, std::move(zeroC), {}, z);
@@ -1200,13 +1393,36 @@ public:
         }
         build_all_merged();
     }
+    // The sync programs of the groups and of the pairs that the step syncs
+    // together.  The groups of the resistive correction are left to their first
+    // use where there is no correction.
     void build_all_merged() {
         mprog.clear();
-        for (int gid = 0; gid < G_NGROUP; ++gid) build_merged(1u << gid);
-        build_merged(MG_EDGE_PAIR);
-        build_merged(MG_STATE_PAIR);
-        build_merged(MG_DERIVED_PAIR);
-        build_merged(MG_PREPARE_PAIR);
+        std::vector<int> todo;
+        for (int gid = 0; gid < G_NGROUP; ++gid)
+            if (P.resist_enabled != 0.0 || (gid != G_ERES && gid != G_ERES0 && gid != G_DB)) todo.push_back(gid);
+        // the groups are independent: a few threads, each with a table of its own
+        std::vector<SyncPlan::Host> h[G_NGROUP];
+        std::atomic<size_t> next{0};
+        auto work = [&] {
+            SyncPlan plan(F->Vtot);
+            for (size_t t; (t = next++) < todo.size();) h[todo[t]] = plan_group(plan, todo[t]);
+        };
+        std::vector<std::future<void>> pool;
+        if (F->Vtot > 100000)
+            for (int t = 0; t < 3; ++t) pool.push_back(std::async(std::launch::async, work));
+        work();
+        for (auto &f : pool) f.get();
+        for (int gid : todo) upload_prog(mprog[1u << gid], h[gid]);
+        for (unsigned pair : {MG_EDGE_PAIR, MG_STATE_PAIR, MG_DERIVED_PAIR, MG_PREPARE_PAIR}) {
+            std::vector<SyncPlan::Host> both;
+            for (int gid = 0; gid < G_NGROUP; ++gid) {
+                if (!(pair & (1u << gid))) continue;
+                if (both.size() < h[gid].size()) both.resize(h[gid].size());
+                for (size_t n = 0; n < h[gid].size(); ++n) both[n].append(h[gid][n]);
+            }
+            upload_prog(mprog[pair], both);
+        }
     }
 
     // the group's copies of one stage (0: halo, 1: owner -> alias) as
@@ -1394,90 +1610,55 @@ public:
     static constexpr unsigned MG_DERIVED_PAIR = (1u << G_BCELL) | (1u << G_JEDGE);
     static constexpr unsigned MG_PREPARE_PAIR = (1u << G_BADD) | (1u << G_BFACE);
 
-    static constexpr size_t kWave = 64;  // wavefront width of gfx950
     static constexpr int kPhaseHalo = 4, kPhaseOwner = 5;  // phases of a group's program (A, B, C, D, H, E)
-    void build_merged(unsigned gset) {
-        MergedProg &mp = mprog[gset];
-        const int g = F->blk[0].g;
-        for (int phase = 0; phase < 6; ++phase)
-            for (OpType t : {OP_FILL, OP_SETV, OP_WALLF, OP_COPY}) {
-                std::unique_ptr<MergedOp> m(new MergedOp());
-                m->type = t;
-                int nset = 0;
-                std::vector<int> ent;
-                std::vector<double> val;
-                for (int gid = 0; gid < G_NGROUP; ++gid) {
-                    if (!(gset & (1u << gid))) continue;
-                    // a caller plan stands in for the halo (phase 4) and owner (phase 5) copies
-                    if (caller_plan[gid] && phase >= kPhaseHalo) continue;
-                    for (auto &o : prog[gid].ops) {
+    std::vector<SyncPlan::Host> plan_group(SyncPlan &plan, int gid) {
+        plan.out.clear();
+        for (const GField &gf : group_fields(gid, nspecies())) {
+            std::vector<const SyncOp *> ops;
+            for (int phase = 0; phase < 6; ++phase) {
+                // a caller plan stands in for the halo (phase 4) and owner (phase 5) copies
+                if (caller_plan[gid] && phase >= kPhaseHalo) continue;
+                for (OpType t : {OP_FILL, OP_SETV, OP_WALLF, OP_COPY})
+                    for (const auto &o : prog[gid].ops) {
                         if (o->phase != phase || o->type != t) continue;
-                        if (t == OP_COPY || t == OP_FILL) {
-                            if (nset >= MERC_MAX_SETS) throw std::runtime_error("merged sync: too many slot sets");
-                            m->S.n[nset] = (int)o->slots.size();
-                            for (size_t c = 0; c < o->slots.size(); ++c) {
-                                m->S.s[nset][c] = o->slots[c];
-                                m->S.v[nset][c] = t == OP_FILL ? o->fillv[c] : 0.0;
+                        for (int sl : o->slots)
+                            if (sl >= gf.slot && sl < gf.slot + gf.ncomp) {
+                                ops.push_back(o.get());
+                                break;
                             }
-                        }
-                        // each op's entries are padded to whole wavefronts with
-                        // entries that do nothing (dst < 0), so that the kernels can
-                        // take the op's slot set as uniform over a wave
-                        const size_t width = t == OP_COPY ? 3 : (t == OP_WALLF ? 4 + g : 2);
-                        if (t == OP_COPY) {
-                            for (size_t e = 0; e + 1 < o->hidx.size(); e += 2) ent.insert(ent.end(), {o->hidx[e], o->hidx[e + 1], nset});
-                            while ((ent.size() / width) % kWave) ent.insert(ent.end(), {-1, -1, nset});
-                        } else if (t == OP_FILL) {
-                            for (int d : o->hidx) ent.insert(ent.end(), {d, nset});
-                            while ((ent.size() / width) % kWave) ent.insert(ent.end(), {-1, nset});
-                        } else if (t == OP_SETV) {
-                            for (size_t e = 0; e < o->hidx.size(); ++e) {
-                                ent.insert(ent.end(), {o->hidx[e], o->slots[0]});
-                                val.push_back(o->hval[e]);
-                            }
-                            while ((ent.size() / width) % kWave) {
-                                ent.insert(ent.end(), {-1, o->slots[0]});
-                                val.push_back(0.0);
-                            }
-                        } else {
-                            const size_t w = 2 + g;
-                            for (size_t e = 0; e + w <= o->hidx.size(); e += w) {
-                                ent.push_back(o->slots[0]);
-                                ent.push_back(o->is_na);
-                                ent.insert(ent.end(), o->hidx.begin() + e, o->hidx.begin() + e + w);
-                            }
-                            while ((ent.size() / width) % kWave) {
-                                ent.push_back(o->slots[0]);
-                                ent.push_back(o->is_na);
-                                ent.insert(ent.end(), w, -1);
-                            }
-                        }
-                        ++nset;
                     }
-                }
-                if (ent.empty()) continue;
-                const int width = t == OP_COPY ? 3 : (t == OP_WALLF ? 4 + g : 2);
-                m->n = (long long)ent.size() / width;
-                m->ent.upload(ent);
-                if (!val.empty()) m->val.upload(val);
-                mp.ops.push_back(std::move(m));
             }
+            plan.add(ops, gf.slot, gf.ncomp, F->blk[0].g);
+        }
+        return std::move(plan.out);
+    }
+    static void upload_prog(SyncProg &p, const std::vector<SyncPlan::Host> &h) {
+        std::vector<double> buf;
+        std::vector<std::array<size_t, 3>> at;
+        auto put = [&](const void *src, size_t bytes) {
+            const size_t o = buf.size();
+            buf.resize(o + (bytes + sizeof(double) - 1) / sizeof(double));
+            if (bytes) std::memcpy(buf.data() + o, src, bytes);
+            return o;
+        };
+        for (const SyncPlan::Host &x : h)
+            at.push_back({put(x.waves.data(), sizeof(SyncWave) * x.waves.size()), put(x.ent.data(), sizeof(int) * x.ent.size()),
+                          put(x.val.data(), sizeof(double) * x.val.size())});
+        p.mem.upload(buf);
+        for (size_t n = 0; n < h.size(); ++n)
+            p.launches.push_back(SyncLaunch{reinterpret_cast<const SyncWave *>(p.mem.p + at[n][0]), (long long)h[n].waves.size(),
+                                            reinterpret_cast<const int *>(p.mem.p + at[n][1]), p.mem.p + at[n][2]});
     }
 
     void run_merged(unsigned gset) { run_merged(gset, st); }
     void run_merged(unsigned gset, hipStream_t s) {
         auto it = mprog.find(gset);
-        if (it == mprog.end()) throw std::runtime_error("merged sync program missing");
-        const int g = F->blk[0].g;
-        for (auto &m : it->second.ops) {
-            switch (m->type) {
-            case OP_COPY: launch_copy_multi(s, m->ent.p, m->n, Fd(), m->S); break;
-            case OP_FILL: launch_fill_multi(s, m->ent.p, m->n, Fd(), m->S); break;
-            case OP_SETV: launch_setv_multi(s, m->ent.p, m->val.p, m->n, Fd()); break;
-            case OP_WALLF: launch_wall_multi(s, m->ent.p, m->n, g, Fd(), P); break;
-            default: break;
-            }
+        if (it == mprog.end()) {  // a group of the resistive correction, by name, without the correction
+            SyncPlan plan(F->Vtot);
+            upload_prog(mprog[gset], plan_group(plan, __builtin_ctz(gset)));
+            it = mprog.find(gset);
         }
+        for (const SyncLaunch &l : it->second.launches) launch_sync(s, l.waves, l.nw, l.ent, l.val, Fd(), P);
         // caller plans: the halo stage of every group of the set, then the owner stage
         for (int t = 0; t < 2; ++t)
             for (int gid = 0; gid < G_NGROUP; ++gid)

@@ -43,10 +43,8 @@ void launch_divb(hipStream_t st, const RangeH &R, const MercBlk *B, double *cons
 void launch_alias_reduce(hipStream_t st, const int *cls_start, const int *member, const int *msign, const int *maxis, const int *owner,
                          const int *osign, const int *oaxis, long long ncls, double *const *F, int slot0);
 void launch_zero_span(hipStream_t st, double *const *F, const int *slots, int ns, long long n);
-void launch_copy_multi(hipStream_t st, const int *ent, long long n, double *const *F, const MultiSets &S);
-void launch_fill_multi(hipStream_t st, const int *ent, long long n, double *const *F, const MultiSets &S);
-void launch_setv_multi(hipStream_t st, const int *ent, const double *val, long long n, double *const *F);
-void launch_wall_multi(hipStream_t st, const int *ent, long long n, int g, double *const *F, const MercPhys &P);
+// one launch of a sync program: nw waves of 64 entries (ent: dst, src per entry)
+void launch_sync(hipStream_t st, const SyncWave *waves, long long nw, const int *ent, const double *val, double *const *F, const MercPhys &P);
 // n entries (dst slot, dst, src slot, src, sign): dst <- sign * src
 void launch_copy_plan(hipStream_t st, const int *ent, long long n, double *const *F);
 // the same entries with every read before every write (sources that are also

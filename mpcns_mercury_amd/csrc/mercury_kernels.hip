@@ -606,42 +606,76 @@ __global__ void k_rk2(const MercRange R, const MercBlk *__restrict__ B, double *
 // ---------------------------------------------------------------------------
 // synchronisation ops (halo / physical boundary / owner-alias), all index lists
 // ---------------------------------------------------------------------------
-// Every entry names its slot set, so one launch serves the lists of several
-// fields (and of independent sync groups). Within one launch no destination is
-// the source of another entry.
-// COPY: entry (dst, src, set), dst <- src for every slot of the set
-// The entry lists of the merged programs are padded per slot set to whole
-// wavefronts (entries with dst < 0 do nothing), so the set, and with it every
-// slot and slot pointer, is uniform over a wave: read once into scalar
-// registers instead of a per-lane chain of table loads before each copy.
-__global__ void k_copy_multi(const int *__restrict__ ent, long long n, double *const *__restrict__ F_, const MultiSets S) {
-    gdouble *const *__restrict__ F = gslots(F_);
-    const long long t = TID;
-    if (t >= n) return;
-    const int d = ent[3 * t], s = ent[3 * t + 1];
-    const int k = __builtin_amdgcn_readfirstlane(ent[3 * t + 2]);
-    if (d < 0) return;
-    for (int c = 0; c < S.n[k]; ++c) F[S.s[k][c]][d] = F[S.s[k][c]][s];
+// A sync (halo, physical boundaries, owner -> alias) is one launch: the host
+// follows the reference's phases symbolically and leaves, for every value that
+// the sync changes, where it comes from among the values before the sync (see
+// SyncPlan in mercury_host.cpp).  Every wave has one kind of entry and one field,
+// so its slots and their pointers are scalar, and a lane reads all components of
+// its source before it writes one: one memory latency per entry.  Bound by launch
+// latency on small blocks (one launch in place of two to five, 7.0 -> 3.6 us per
+// edge sync of a 48^3 block) and by scattered 32-byte writes on large ones (state
+// sync of the 2.53 M-cell shell 33 -> 25 us, of a 16-run ensemble 93 -> 35 us).
+template <int NC>
+DEVI void sync_copy(gdouble *const *__restrict__ F, int slot, int d, int s) {
+    double v[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) v[c] = F[slot + c][s];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) F[slot + c][d] = v[c];
 }
-// FILL: entry (dst, set), dst <- the set's constant per slot
-__global__ void k_fill_multi(const int *__restrict__ ent, long long n, double *const *__restrict__ F_, const MultiSets S) {
+struct WallParams {
+    double gm1, p_floor, rho_floor[MERC_NSMAX];
+};
+__global__ void __launch_bounds__(256) k_sync(const SyncWave *__restrict__ waves, long long nw, const int2 *__restrict__ ent,
+                                              const double *__restrict__ val, double *const *__restrict__ F_, const WallParams P) {
     gdouble *const *__restrict__ F = gslots(F_);
-    const long long t = TID;
-    if (t >= n) return;
-    const int d = ent[2 * t];
-    const int k = __builtin_amdgcn_readfirstlane(ent[2 * t + 1]);
-    if (d < 0) return;
-    for (int c = 0; c < S.n[k]; ++c) F[S.s[k][c]][d] = S.v[k][c];
-}
-// SETV: entry (dst, slot) with its own value
-__global__ void k_setv_multi(const int *__restrict__ ent, const double *__restrict__ val, long long n, double *const *__restrict__ F_) {
-    gdouble *const *__restrict__ F = gslots(F_);
-    const long long t = TID;
-    if (t >= n) return;
-    const int d = ent[2 * t];
-    const int slot = __builtin_amdgcn_readfirstlane(ent[2 * t + 1]);
-    if (d < 0) return;
-    F[slot][d] = val[t];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)(TID >> 6));
+    if (w >= nw) return;
+    const SyncWave W = waves[w];
+    const int2 e = ent[(long long)W.first + lane];
+    const int d = e.x, s = e.y;
+    if (d < 0) return;  // padding to whole waves
+    const int slot = W.slot;
+    if (W.kind == SYNC_COPY) {
+        if (W.ncomp == 1) sync_copy<1>(F, slot, d, s);
+        else if (W.ncomp == 3) sync_copy<3>(F, slot, d, s);
+        else sync_copy<5>(F, slot, d, s);
+    } else if (W.kind == SYNC_CONST) {
+        for (int c = 0; c < W.ncomp; ++c) F[slot + c][d] = val[s + c];
+    } else if (W.kind == SYNC_CHAIN) {
+        for (int c = 0; c < W.ncomp; ++c) {
+            const double old = F[slot + c][d], owner = F[slot + c][s];
+            for (int u = 1; u <= W.np; ++u) {
+                const int2 g = ent[(long long)W.first + 64 * u + lane];
+                if (g.x >= 0) F[slot + c][g.x] = old;
+                if (g.y >= 0) F[slot + c][g.y] = old;
+            }
+            F[slot + c][d] = owner;
+        }
+    } else {
+        // BC_Solid_Surface_ (Boundary_Condition_Fluid.cpp:36-260), H+ (He++ takes
+        // the same rule with its own density floor): first layer from the cell
+        // behind it, ghosts from the first layer
+        double v[5];
+#pragma unroll
+        for (int m = 0; m < 5; ++m) v[m] = F[slot + m][s];
+        const double rho_floor = P.rho_floor[W.species];
+        for (int n = W.kind == SYNC_WALL2 ? 2 : 1; n > 0; --n) {
+            const double rho_r = dmax(v[0], rho_floor);
+            const double rho2 = dmax(rho_r, rho_floor);
+            const double ke = 0.5 * (v[1] * v[1] + v[2] * v[2] + v[3] * v[3]) / rho2;
+            double eint = v[4] - ke;
+            if (eint < 0.0) eint = 0.0;
+            const double p_r = dmax(P.gm1 * eint, P.p_floor);
+            const double ke_g = 0.5 * rho_r * 0.0;
+            v[0] = rho_r;
+            v[1] = v[2] = v[3] = rho_r * 0.0;
+            v[4] = p_r / P.gm1 + ke_g;
+        }
+#pragma unroll
+        for (int m = 0; m < 5; ++m) F[slot + m][d] = v[m];
+    }
 }
 // a caller's sync plan: entry (dst slot, dst, src slot, src, sign), dst <- sign * src
 __global__ void k_copy_plan(const int *__restrict__ ent, long long n, double *const *__restrict__ F_) {
@@ -667,51 +701,6 @@ __global__ void k_plan_scatter(const int *__restrict__ ent, long long n, double 
     const int *e = ent + 5 * t;
     F[e[0]][e[1]] = tmp[t];
 }
-// BC_Solid_Surface_ (Boundary_Condition_Fluid.cpp:36-260): per wall cell the
-// entry holds (species base slot, species (0 H+, 1 Na+, 2 He++), first layer,
-// one deeper, g ghosts); He++ takes the H+ rule with its own density floor
-__global__ void k_wall_multi(const int *__restrict__ ent, long long n, int g, double *const *__restrict__ F_, const MercPhys P) {
-    gdouble *const *__restrict__ F = gslots(F_);
-    const long long t = TID;
-    if (t >= n) return;
-    const int *e = ent + (long long)t * (4 + g);
-    const int slot = __builtin_amdgcn_readfirstlane(e[0]), species = __builtin_amdgcn_readfirstlane(e[1]), is_na = species == 1;
-    e += 2;
-    if (e[0] < 0) return;  // padding of the entry list to whole waves
-    const double gm1 = P.gamma - 1.0;
-    const double rho_floor = species == 1 ? P.wall_rho_floor_Na : (species == 2 ? P.wall_rho_floor_He : P.wall_rho_floor_H);
-    const double p_floor = P.wall_p_floor;
-    if (is_na) {
-        for (int l = 0; l < g; ++l) {
-            const int d = e[2 + l];
-            F[slot][d] = rho_floor;
-            F[slot + 1][d] = 0.0;
-            F[slot + 2][d] = 0.0;
-            F[slot + 3][d] = 0.0;
-            F[slot + 4][d] = p_floor / gm1;
-        }
-        return;
-    }
-    for (int layer = 0; layer <= g; ++layer) {
-        const int r = layer == 0 ? e[1] : e[0];
-        const int d = layer == 0 ? e[0] : e[1 + layer];
-        const double rho_r = dmax(F[slot][r], rho_floor);
-        const double mxr = F[slot + 1][r], myr = F[slot + 2][r], mzr = F[slot + 3][r];
-        const double Er = F[slot + 4][r];
-        const double rho2 = dmax(rho_r, rho_floor);
-        const double ke = 0.5 * (mxr * mxr + myr * myr + mzr * mzr) / rho2;
-        double eint = Er - ke;
-        if (eint < 0.0) eint = 0.0;
-        const double p_r = dmax(gm1 * eint, p_floor);
-        F[slot][d] = rho_r;
-        F[slot + 1][d] = rho_r * 0.0;
-        F[slot + 2][d] = rho_r * 0.0;
-        F[slot + 3][d] = rho_r * 0.0;
-        const double ke_g = 0.5 * rho_r * 0.0;
-        F[slot + 4][d] = p_r / gm1 + ke_g;
-    }
-}
-
 // owner <- signed mean of an equivalence class (ReduceEdgeAliasCandidatesToOwners_,
 // MercurySolver_Current.cpp:3-57); members summed in the listed order, each
 // read from the triplet field of its own axis
@@ -836,9 +825,10 @@ __global__ void __launch_bounds__(256) k_divb_final(const double *__restrict__ p
     }
 }
 
+constexpr int kZeroSlots = 10;
 struct SlotSet {
     int n;
-    int s[MERC_MAX_SYNC_SLOTS];
+    int s[kZeroSlots];
 };
 // zero a set of slots over whole blocks (replaces memset inside a captured step)
 __global__ void k_zero_span(double *const *__restrict__ F_, const SlotSet S, long long n) {
@@ -919,14 +909,10 @@ void launch_alias_reduce(hipStream_t st, const int *cls_start, const int *member
         hipLaunchKernelGGL(k_alias_reduce, dim3(nblk(ncls, 256)), dim3(256), 0, st, cls_start, member, msign, maxis, owner, osign, oaxis, ncls,
                            F, slot0);
 }
-void launch_copy_multi(hipStream_t st, const int *ent, long long n, double *const *F, const MultiSets &S) {
-    if (n > 0) hipLaunchKernelGGL(k_copy_multi, dim3(nblk(n, 256)), dim3(256), 0, st, ent, n, F, S);
-}
-void launch_fill_multi(hipStream_t st, const int *ent, long long n, double *const *F, const MultiSets &S) {
-    if (n > 0) hipLaunchKernelGGL(k_fill_multi, dim3(nblk(n, 256)), dim3(256), 0, st, ent, n, F, S);
-}
-void launch_setv_multi(hipStream_t st, const int *ent, const double *val, long long n, double *const *F) {
-    if (n > 0) hipLaunchKernelGGL(k_setv_multi, dim3(nblk(n, 256)), dim3(256), 0, st, ent, val, n, F);
+void launch_sync(hipStream_t st, const SyncWave *waves, long long nw, const int *ent, const double *val, double *const *F, const MercPhys &P) {
+    if (nw <= 0) return;
+    const WallParams wp = {P.gamma - 1.0, P.wall_p_floor, {P.wall_rho_floor_H, P.wall_rho_floor_Na, P.wall_rho_floor_He}};
+    hipLaunchKernelGGL(k_sync, dim3(nblk(nw, 4)), dim3(256), 0, st, waves, nw, reinterpret_cast<const int2 *>(ent), val, F, wp);
 }
 void launch_copy_plan(hipStream_t st, const int *ent, long long n, double *const *F) {
     if (n > 0) hipLaunchKernelGGL(k_copy_plan, dim3(nblk(n, 256)), dim3(256), 0, st, ent, n, F);
@@ -935,9 +921,6 @@ void launch_copy_plan_staged(hipStream_t st, const int *ent, long long n, double
     if (n <= 0) return;
     hipLaunchKernelGGL(k_plan_gather, dim3(nblk(n, 256)), dim3(256), 0, st, ent, n, F, tmp);
     hipLaunchKernelGGL(k_plan_scatter, dim3(nblk(n, 256)), dim3(256), 0, st, ent, n, F, (const double *)tmp);
-}
-void launch_wall_multi(hipStream_t st, const int *ent, long long n, int g, double *const *F, const MercPhys &P) {
-    if (n > 0) hipLaunchKernelGGL(k_wall_multi, dim3(nblk(n, 256)), dim3(256), 0, st, ent, n, g, F, P);
 }
 void launch_zero_span(hipStream_t st, double *const *F, const int *slots, int ns, long long n) {
     if (n <= 0) return;
