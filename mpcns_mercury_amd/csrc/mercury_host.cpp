@@ -885,6 +885,8 @@ public:
     RangeOwner R_res;  // node-box points around the resistive unknowns (the CG's curls)
     RangeOwner R_march;  // flux pass: ceil(m0 / march) x m1 x m2 per block (column kernel)
     int march = 4;       // owned cells per thread along i in the flux pass
+    bool march_auto = true;  // by auto_march (until the caller, the autotuner or the environment chooses)
+    int simds = 1024;        // of the device
     RangeOwner R_tile;   // tiled flux pass: ceil(m0 / tile_c) x ceil(m1 / 16) x ceil(m2 / 16) tiles per block
     int tile_c = 0;      // planes per tile along i; 0: the column kernel runs
     GroupProg prog[G_NGROUP];
@@ -1124,15 +1126,26 @@ public:
         make_range(*F, 0, 1, R_node);
         HIPCHK(hipMalloc(&d_mpart, 2 * sizeof(double) * (size_t)std::max<long long>((R_node.h.total + 255) / 256, 1)));
         make_range(*F, -1, 2, R_eface);
-        if (const char *e = std::getenv("MERCURY_RHS_MARCH")) march = std::max(1, std::atoi(e));
-        if (const char *e = std::getenv("MERCURY_RHS_TILE")) tile_c = std::max(0, std::atoi(e));
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+            simds = 4 * cus;
+        march = auto_march();
+        if (const char *e = std::getenv("MERCURY_RHS_MARCH")) march = std::max(1, std::atoi(e)), march_auto = false;
+        if (const char *e = std::getenv("MERCURY_RHS_TILE")) tile_c = std::max(0, std::atoi(e)), march_auto = false;
+        // Two streams pay where the passes are long: a step of 2.1 M cells takes
+        // 1410 us with and 1428 without (FP64), of 512 k cells 417 either way; the
+        // forks and joins cost a short one more than they bring (204 k cells 219
+        // against 215 us, mixed 166 / 157; 48^3 147 / 132; 12x10x8 98 / 74).
+        long long cells = 0;
+        for (const MercBlk &k : F->blk) cells += (long long)k.m[0] * k.m[1] * k.m[2];
+        overlap = cells >= (1LL << 19);
         if (const char *e = std::getenv("MERCURY_OVERLAP")) overlap = std::atoi(e) != 0;
         HIPCHK(hipStreamCreateWithFlags(&st2, hipStreamNonBlocking));
         HIPCHK(hipEventCreateWithFlags(&ev_fork, hipEventDisableTiming));
         HIPCHK(hipEventCreateWithFlags(&ev_join, hipEventDisableTiming));
         HIPCHK(hipEventCreateWithFlags(&ev_fork2, hipEventDisableTiming));
         HIPCHK(hipEventCreateWithFlags(&ev_join2, hipEventDisableTiming));
-        set_flux_shape(tile_c > 0 ? 1 : 0, tile_c > 0 ? tile_c : march);
+        apply_flux_shape(tile_c > 0 ? 1 : 0, tile_c > 0 ? tile_c : march);
         cls.build(*F);
         build_programs();
         alias.build(cls);
@@ -1206,6 +1219,26 @@ public:
     // along i for the column kernel, L planes per 16 x 16 tile for the tiled
     // one; drops a captured step graph (it holds the old shape)
     void set_flux_shape(int kind, int L) {
+        apply_flux_shape(kind, L);
+        march_auto = false;
+    }
+    // Cells per thread along i of the column kernel when nobody chose: 4 share
+    // the most work (the i flux and the neighbour planes), as long as the waves
+    // fill the chip several times over; the kernel keeps two waves per SIMD in
+    // FP64 and three in the mixed form, and with fewer than four rounds of them
+    // the last round and the longer serial chain cost more.  Measured at 4, 2, 1
+    // cells: 2.53 M cells FP64 360, 367, 387 us and mixed 273, 271, 281; 546 k
+    // cells 120, 107, 105 and 83, 75, 68; 48^3 34, 20, 19; 12x10x8 26, 15, 10.
+    int auto_march() const {
+        const long long need = 4LL * simds * (form == 2 ? 3 : 2);
+        for (int L : {4, 2}) {
+            long long waves = 0;
+            for (const MercBlk &k : F->blk) waves += (long long)((k.m[0] + L - 1) / L) * k.m[1] * k.m[2];
+            if (waves / 64 >= need) return L;
+        }
+        return 1;
+    }
+    void apply_flux_shape(int kind, int L) {
         if (L < 1) throw std::runtime_error("mercury_set_flux_shape: length must be >= 1");
         if (kind < 0 || kind > 1) throw std::runtime_error("mercury_set_flux_shape: kind must be 0 (column) or 1 (tiled)");
         ++generation;
@@ -2179,6 +2212,7 @@ public:
         if (f == form) return;
         form = f;
         ++generation;
+        if (march_auto) apply_flux_shape(0, auto_march());
         if (f >= 1 && prepared) {
             refresh_float_statics();
             derived_fused(true);
