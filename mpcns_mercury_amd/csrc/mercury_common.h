@@ -125,12 +125,12 @@ enum MercBC { MBC_PERIODIC = 0, MBC_FARFIELD = 1, MBC_WALL = 2, MBC_INTERFACE = 
 // WALL2: the reflected state at a solid surface, once (the first layer) or twice
 // (the ghosts, made from the first layer) over the state at src, the cell behind
 // the first layer.  CHAIN: dst is an aliased value that goes to up to 2 np ghosts
-// before its owner's value, src, replaces it; the ghosts follow, two to an entry,
-// the n-th pair of a lane 64 n entries further.
-enum SyncKind { SYNC_COPY = 0, SYNC_CONST, SYNC_WALL1, SYNC_WALL2, SYNC_CHAIN };
+// before its owner's value, src, replaces it (CHAIN_CONST: the values at src); the
+// ghosts follow, two to an entry, the n-th pair of a lane 64 n entries further.
+enum SyncKind { SYNC_COPY = 0, SYNC_CONST, SYNC_WALL1, SYNC_WALL2, SYNC_CHAIN, SYNC_CHAIN_CONST };
 struct SyncWave {
     int kind, slot, ncomp;
     int first;    // first entry
     int species;  // WALL1, WALL2: 0 H+, 2 He++
-    int np;       // CHAIN: pairs of ghosts
+    int np;       // CHAIN, CHAIN_CONST: pairs of ghosts
 };

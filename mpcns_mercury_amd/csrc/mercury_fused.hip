@@ -910,7 +910,18 @@ __global__ void k_edge_total(const MercRange R, const MercBlk *__restrict__ B, d
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
         if (idx[a] >= bk.m[a]) continue;
-        F[SL_E + a][q] = (double)E[a];
+        double e = (double)E[a];
+        if (with_hall == 3) {
+            bool shared = false, wall = false;
+            for (int f = 0; f < 6; ++f) {
+                const int nax = f >> 1;
+                if (nax == a || ((f & 1) ? (idx[nax] != bk.m[nax]) : (idx[nax] != 0))) continue;
+                shared |= bk.bc[f] == MBC_PERIODIC || bk.bc[f] == MBC_INTERFACE;
+                wall |= bk.bc[f] == MBC_WALL;
+            }
+            if (!shared) e = wall ? 0.0 : e + (double)hall[a];
+        }
+        F[SL_E + a][q] = e;
         if (with_hall) F[SL_EH + a][q] = (double)hall[a];
     }
 #undef FB

@@ -212,8 +212,7 @@ public:
     }
     // (block, i, j, k) of an arena index (the inverse of gidx)
     void point_of(int x, int p[4]) const {
-        int b = 0;
-        while (b + 1 < nb() && blk[b + 1].off <= x) ++b;
+        const int b = (int)(std::upper_bound(blk.begin(), blk.end(), (long long)x, [](long long v, const MercBlk &k) { return v < k.off; }) - blk.begin()) - 1;
         const MercBlk &q = blk[b];
         long long r = x - q.off;
         p[0] = b;
@@ -370,7 +369,7 @@ public:
             val.insert(val.end(), o.val.begin(), o.val.end());
             for (SyncWave w : o.waves) {
                 w.first += e0;
-                if (w.kind == SYNC_CONST)
+                if (w.kind == SYNC_CONST || w.kind == SYNC_CHAIN_CONST)
                     for (int l = 0; l < 64; ++l) ent[2 * ((size_t)w.first + l) + 1] += v0;
                 waves.push_back(w);
             }
@@ -455,8 +454,8 @@ private:
         };
         for (const auto &p : chain) {
             const Sym v = sym[p.first];
-            // the value read is replaced by an unchanged one, and the reader is read by nobody
-            if (v.type != RAW || sym[v.a].type != NONE || read(p.second)) return false;
+            // the value read is replaced by an unchanged one or a constant, and the reader is read by nobody
+            if ((v.type != CST && (v.type != RAW || sym[v.a].type != NONE)) || read(p.second)) return false;
         }
         return true;
     }
@@ -468,12 +467,12 @@ private:
         H.val.insert(H.val.end(), rows.begin(), rows.end());
         for (int d : touched) {
             const Sym v = sym[d];
+            if (!chain.empty()) {
+                const auto it = std::lower_bound(chain.begin(), chain.end(), std::make_pair(d, INT_MIN));
+                if (it != chain.end() && it->first == d) continue;  // the end of a chain
+            }
             if (v.type == RAW) {
-                if (v.a == d || sym[v.a].type != NONE) continue;  // unchanged, or part of a chain
-                if (!chain.empty()) {
-                    const auto it = std::lower_bound(chain.begin(), chain.end(), std::make_pair(d, INT_MIN));
-                    if (it != chain.end() && it->first == d) continue;  // the end of a chain
-                }
+                if (v.a == d || sym[v.a].type != NONE) continue;  // unchanged, or a reader in a chain
                 part[SYNC_COPY].insert(part[SYNC_COPY].end(), {d, v.a});
             } else if (v.type == CST) {
                 part[SYNC_CONST].insert(part[SYNC_CONST].end(), {d, base + v.a});
@@ -490,24 +489,26 @@ private:
                 H.ent.resize(H.ent.size() + 2 * kWaveEntries - n, -1);
             }
         // chains, 64 a wave: (aliased value, owner), then the ghosts that read it
-        std::vector<std::pair<int, int>> lane;  // (number of ghosts, first in chain), the short ones first
-        for (size_t t = 0, u; t < chain.size(); t = u) {
-            for (u = t + 1; u < chain.size() && chain[u].first == chain[t].first;) ++u;
-            lane.push_back({(int)(u - t), (int)t});
-        }
-        std::sort(lane.begin(), lane.end());
-        for (size_t t = 0; t < lane.size(); t += kWaveEntries) {
-            const size_t n = std::min(kWaveEntries, lane.size() - t);
-            const int np = (lane[t + n - 1].first + 1) / 2;
-            H.waves.push_back(SyncWave{SYNC_CHAIN, slot, ncomp, (int)(H.ent.size() / 2), 0, np});
-            const size_t e0 = H.ent.size();
-            H.ent.resize(e0 + 2 * kWaveEntries * (1 + np), -1);
-            for (size_t l = 0; l < n; ++l) {
-                const auto &c = lane[t + l];
-                const int x = chain[c.second].first;
-                H.ent[e0 + 2 * l] = x;
-                H.ent[e0 + 2 * l + 1] = sym[x].a;
-                for (int u = 0; u < c.first; ++u) H.ent[e0 + 2 * (kWaveEntries * (1 + u / 2) + l) + u % 2] = chain[c.second + u].second;
+        for (int kind : {SYNC_CHAIN, SYNC_CHAIN_CONST}) {
+            std::vector<std::pair<int, int>> lane;  // (number of ghosts, first in chain), the short ones first
+            for (size_t t = 0, u; t < chain.size(); t = u) {
+                for (u = t + 1; u < chain.size() && chain[u].first == chain[t].first;) ++u;
+                if ((sym[chain[t].first].type == CST) == (kind == SYNC_CHAIN_CONST)) lane.push_back({(int)(u - t), (int)t});
+            }
+            std::sort(lane.begin(), lane.end());
+            for (size_t t = 0; t < lane.size(); t += kWaveEntries) {
+                const size_t n = std::min(kWaveEntries, lane.size() - t);
+                const int np = (lane[t + n - 1].first + 1) / 2;
+                H.waves.push_back(SyncWave{kind, slot, ncomp, (int)(H.ent.size() / 2), 0, np});
+                const size_t e0 = H.ent.size();
+                H.ent.resize(e0 + 2 * kWaveEntries * (1 + np), -1);
+                for (size_t l = 0; l < n; ++l) {
+                    const auto &c = lane[t + l];
+                    const int x = chain[c.second].first;
+                    H.ent[e0 + 2 * l] = x;
+                    H.ent[e0 + 2 * l + 1] = sym[x].a + (kind == SYNC_CHAIN_CONST ? base : 0);
+                    for (int u = 0; u < c.first; ++u) H.ent[e0 + 2 * (kWaveEntries * (1 + u / 2) + l) + u % 2] = chain[c.second + u].second;
+                }
             }
         }
         reset();
@@ -793,6 +794,8 @@ struct Classes {
 // lives in); per class the owner's index, sign and axis
 struct AliasClasses {
     DBuf<int> start, member, msign, maxis, owner, osign, oaxis;
+    DBuf<int> wall;    // per member: an edge of a solid surface (own classes)
+    bool own = false;  // the classes of the blocks' own connections: one axis and sign +1 each
     long long n = 0;
     // host copies (arena indices), for the export and the resistive unknowns
     std::vector<int> hst{0}, hmem, hms, hmax, how, hos, hoax;
@@ -813,8 +816,9 @@ struct AliasClasses {
         how = std::move(ow);
         hos = std::move(os);
         hoax = std::move(oax);
+        own = false;
     }
-    void build(const Classes &C) {
+    void build(const Classes &C, const Field &F) {
         std::vector<int> st{0}, mem, ms, max, ow, os, oax;
         for (int a = 0; a < 3; ++a) {
             const int L = LOC_EX + a;
@@ -831,6 +835,17 @@ struct AliasClasses {
             }
         }
         set(std::move(st), std::move(mem), std::move(ms), std::move(max), std::move(ow), std::move(os), std::move(oax));
+        std::vector<int> w;
+        for (size_t t = 0; t < hmem.size(); ++t) {
+            int p[4];
+            F.point_of(hmem[t], p);
+            const MercBlk &k = F.blk[p[0]];
+            bool on = false;
+            for (int f = 0; f < 6; ++f) on |= k.bc[f] == MBC_WALL && f / 2 != hmax[t] && p[1 + f / 2] == ((f & 1) ? k.m[f / 2] : 0);
+            w.push_back(on);
+        }
+        wall.upload(w);
+        own = true;
     }
     // non-owner members of each axis (arena index flags)
     void alias_flags(long long V, std::vector<char> flags[3]) const {
@@ -838,6 +853,9 @@ struct AliasClasses {
         for (size_t c = 0; c + 1 < hst.size(); ++c)
             for (int t = hst[c]; t < hst[c + 1]; ++t)
                 if (!(hmem[t] == how[c] && hmax[t] == hoax[c])) flags[hmax[t]][hmem[t]] = 1;
+    }
+    void launch_emf(hipStream_t st, double *const *F) const {
+        launch_alias_emf(st, start.p, member.p, maxis.p, wall.p, owner.p, n, F);
     }
     void launch(hipStream_t st, double *const *F, int slot0) const {
         launch_alias_reduce(st, start.p, member.p, msign.p, maxis.p, owner.p, osign.p, oaxis.p, n, F, slot0);
@@ -1148,7 +1166,7 @@ public:
         apply_flux_shape(tile_c > 0 ? 1 : 0, tile_c > 0 ? tile_c : march);
         cls.build(*F);
         build_programs();
-        alias.build(cls);
+        alias.build(cls, *F);
         if (ptopo) apply_patch_plans();
         build_resist();
     }
@@ -1953,10 +1971,12 @@ public:
         if (alias.n == 0) {
             launch_edge_total(st, R_node.h, Bd(), Fd(), Gd(), P, 1, mix());
             run_merged(MG_EDGE_PAIR);
-            if (overlap) HIPCHK(hipStreamWaitEvent(st, ev_join, 0));
-            launch_update_all(st, R_node.h, Bd(), Fd(), Gd(), dtp(), mix(), nspecies());
-            after_update(final);
-            return;
+        } else if (alias.own && !any_caller_plan()) {
+            // shared edges of the blocks' own connections: the edge pass leaves
+            // them to one pass over the classes
+            launch_edge_total(st, R_node.h, Bd(), Fd(), Gd(), P, 3, mix());
+            alias.launch_emf(st, Fd());
+            run_merged(MG_EDGE_PAIR);
         } else {
             // shared edges (periodic seams, interfaces): the alias mean of the
             // non-Hall EMF before the Hall part is added; one pass writes both
@@ -1965,8 +1985,8 @@ public:
             singular_emf(mix());
             sync(G_EHALL);
             launch_add_hall_wall(st, R_node.h, Bd(), Fd());
+            sync(G_EEDGE);
         }
-        sync(G_EEDGE);
         if (overlap) HIPCHK(hipStreamWaitEvent(st, ev_join, 0));
         launch_update_all(st, R_node.h, Bd(), Fd(), Gd(), dtp(), mix(), nspecies());
         after_update(final);

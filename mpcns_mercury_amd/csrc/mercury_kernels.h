@@ -43,6 +43,9 @@ void launch_divb(hipStream_t st, const RangeH &R, const MercBlk *B, double *cons
 void launch_alias_reduce(hipStream_t st, const int *cls_start, const int *member, const int *msign, const int *maxis, const int *owner,
                          const int *osign, const int *oaxis, long long ncls, double *const *F, int slot0);
 void launch_zero_span(hipStream_t st, double *const *F, const int *slots, int ns, long long n);
+// classes of one axis and sign each (wall: per member, an edge of a solid surface)
+void launch_alias_emf(hipStream_t st, const int *cls_start, const int *member, const int *axis, const int *wall, const int *owner,
+                      long long ncls, double *const *F);
 // one launch of a sync program: nw waves of 64 entries (ent: dst, src per entry)
 void launch_sync(hipStream_t st, const SyncWave *waves, long long nw, const int *ent, const double *val, double *const *F, const MercPhys &P);
 // n entries (dst slot, dst, src slot, src, sign): dst <- sign * src

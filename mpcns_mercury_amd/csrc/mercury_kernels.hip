@@ -643,9 +643,9 @@ __global__ void __launch_bounds__(256) k_sync(const SyncWave *__restrict__ waves
         else sync_copy<5>(F, slot, d, s);
     } else if (W.kind == SYNC_CONST) {
         for (int c = 0; c < W.ncomp; ++c) F[slot + c][d] = val[s + c];
-    } else if (W.kind == SYNC_CHAIN) {
+    } else if (W.kind == SYNC_CHAIN || W.kind == SYNC_CHAIN_CONST) {
         for (int c = 0; c < W.ncomp; ++c) {
-            const double old = F[slot + c][d], owner = F[slot + c][s];
+            const double old = F[slot + c][d], owner = W.kind == SYNC_CHAIN ? F[slot + c][s] : val[s + c];
             for (int u = 1; u <= W.np; ++u) {
                 const int2 g = ent[(long long)W.first + 64 * u + lane];
                 if (g.x >= 0) F[slot + c][g.x] = old;
@@ -714,6 +714,31 @@ __global__ void k_alias_reduce(const int *__restrict__ cls_start, const int *__r
     double sum = 0.0;
     for (int m = b; m < e; ++m) sum += msign[m] * F[slot0 + maxis[m]][member[m]];
     F[slot0 + oaxis[t]][owner[t]] = osign[t] * sum / (double)(e - b);
+}
+
+// The edges shared between blocks or across a periodic seam, after the edge pass
+// has left their non-Hall and Hall EMFs apart: the owner takes the mean of its
+// class (k_alias_reduce), then every member adds the owner's Hall EMF (which the
+// Ehall sync leaves in each of them) and the stationary wall zeroes its edges
+// (k_add_hall_wall).  One thread per class in place of a pass over all edges
+// behind a sync of its own: a pass of 18 us and a sync of 16 on the 24-block
+// shell of 546 k cells, two launches of 3-4 us on the smallest block.
+__global__ void k_alias_emf(const int *__restrict__ cls_start, const int *__restrict__ member, const int *__restrict__ axis,
+                            const int *__restrict__ wall, const int *__restrict__ owner, long long ncls, double *const *__restrict__ F_) {
+    gdouble *const *__restrict__ F = gslots(F_);
+    const long long t = TID;
+    if (t >= ncls) return;
+    const int b = cls_start[t], e = cls_start[t + 1], o = owner[t];
+    gdouble *E = F[SL_E + axis[b]];
+    const double hall = F[SL_EH + axis[b]][o];
+    double sum = 0.0;
+    for (int m = b; m < e; ++m) sum += 1 * E[member[m]];
+    const double mean = 1 * sum / (double)(e - b);
+    for (int m = b; m < e; ++m) {
+        const int q = member[m];
+        const double v = (q == o ? mean : E[q]) + hall;
+        E[q] = wall[m] ? 0.0 : v;
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -908,6 +933,11 @@ void launch_alias_reduce(hipStream_t st, const int *cls_start, const int *member
     if (ncls > 0)
         hipLaunchKernelGGL(k_alias_reduce, dim3(nblk(ncls, 256)), dim3(256), 0, st, cls_start, member, msign, maxis, owner, osign, oaxis, ncls,
                            F, slot0);
+}
+void launch_alias_emf(hipStream_t st, const int *cls_start, const int *member, const int *axis, const int *wall, const int *owner,
+                      long long ncls, double *const *F) {
+    if (ncls > 0)
+        hipLaunchKernelGGL(k_alias_emf, dim3(nblk(ncls, 256)), dim3(256), 0, st, cls_start, member, axis, wall, owner, ncls, F);
 }
 void launch_sync(hipStream_t st, const SyncWave *waves, long long nw, const int *ent, const double *val, double *const *F, const MercPhys &P) {
     if (nw <= 0) return;

@@ -40,3 +40,27 @@ def test_streams_and_shapes_keep_every_bit(oracle_mod, monkeypatch, overlap, len
                 np.testing.assert_array_equal(g.get(name, ib), o.get(name, ib), err_msg=f"{name}[{ib}]")
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("name", ["cube", "cut_cube", "cut_sector"])
+def test_shared_edges_take_mean_and_hall(oracle_mod, name):
+    """E and the Hall EMF on every owned edge, those shared across a seam or an
+    interface and those that also lie on the solid surface among them."""
+    case = {"cube": lambda: cases.make_periodic_cube(n=(7, 6, 8), g=4, hall=True),
+            "cut_cube": lambda: cases.make_split_cube(n=(9, 8, 10), split=(2, 2, 2), g=4, hall=True),
+            "cut_sector": lambda: cases.make_split_sector(dims=(12, 9, 10), cuts=((5, 7), (4, 5), (10,)))}[name]()
+    g = Mercury(case)
+    o = oracle_mod.Oracle(case)
+    try:
+        g.prepare()
+        o.prepare()
+        np.testing.assert_array_equal(g.step(2), o.step(2))
+        for field in ("E", "Ehall"):
+            for a, axis in enumerate(("xi", "eta", "zeta")):
+                for ib in range(case.nb):
+                    m = case.blocks[ib].dims
+                    own = (slice(None),) + tuple(slice(case.g, case.g + m[c] + (c != a)) for c in range(3))
+                    n = f"{field}_{axis}"
+                    np.testing.assert_array_equal(g.get(n, ib)[own], o.get(n, ib)[own], err_msg=f"{n}[{ib}]")
+    finally:
+        g.close()
