@@ -18,6 +18,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <future>
 #include <initializer_list>
 #include <map>
@@ -251,6 +252,7 @@ struct RangeOwner {
     RangeH h;
     DBuf<long long> start;
     DBuf<int> lo, n;
+    std::vector<int> hlo, hn;  // the boxes, on the host
 };
 
 // per block box [lo, lo + n) (n = 0: no point of the block)
@@ -260,6 +262,8 @@ static void make_range_boxes(const Field &F, const std::vector<int> &lo, const s
     R.start.upload(st);
     R.lo.upload(lo);
     R.n.upload(n);
+    R.hlo = lo;
+    R.hn = n;
     R.h.dev.nb = F.nb();
     R.h.dev.start = R.start.p;
     R.h.dev.lo = R.lo.p;
@@ -283,6 +287,8 @@ static void make_range(const Field &F, int lo_off, int hi_off, RangeOwner &R) {
     R.start.upload(st);
     R.lo.upload(lo);
     R.n.upload(n);
+    R.hlo = lo;
+    R.hn = n;
     R.h.dev.nb = F.nb();
     R.h.dev.start = R.start.p;
     R.h.dev.lo = R.lo.p;
@@ -341,7 +347,8 @@ public:
     explicit SyncPlan(long long nvalues) : sym(nvalues, {NONE, 0}) {}
     // appends one field's sync: ops in program order that touch slots slot ..
     // slot + ncomp - 1; launch n of every field goes to the same kernel launch
-    void add(const std::vector<const SyncOp *> &ops, int slot, int ncomp, int g) {
+    // keep: the values to write (all of them without it)
+    void add(const std::vector<const SyncOp *> &ops, int slot, int ncomp, int g, const std::function<bool(int)> &keep = nullptr) {
         // where a launch may end: not between the components of one set of values
         std::vector<size_t> ends;
         for (size_t n = 0; n < ops.size(); ++n) {
@@ -352,7 +359,7 @@ public:
         for (size_t u = 0; u < ends.size();) {
             size_t last = ends.size() - 1;
             // one op by itself always can: no destination of it is a source of it
-            while (!(follow(ops, at, ends[last], slot, ncomp, g) && joins()) && last > u) --last;
+            while (!(follow(ops, at, ends[last], slot, ncomp, g) && (last + 1 < ends.size() || !keep || drop(keep)) && joins()) && last > u) --last;
             emit(launch++, slot, ncomp);
             at = ends[last];
             u = last + 1;
@@ -436,6 +443,17 @@ private:
                 for (size_t t = 0; t + 1 < o.hidx.size(); t += 2) set(o.hidx[t], value_of(o.hidx[t + 1]));
             }
         }
+        return true;
+    }
+    // drops the values that need not be written (in the last launch of a field, so
+    // that no later op reads them)
+    bool drop(const std::function<bool(int)> &keep) {
+        size_t n = 0;
+        for (int d : touched) {
+            if (keep(d)) touched[n++] = d;
+            else sym[d] = {NONE, 0};
+        }
+        touched.resize(n);
         return true;
     }
     // whether the values can be written in one launch; collects the chains
@@ -981,6 +999,8 @@ public:
     double *rwd = nullptr;  // w / dg, the weight of r.z
     double *rx = nullptr, *rr = nullptr, *rp = nullptr, *rAp = nullptr, *rb = nullptr, *rdg = nullptr, *rw = nullptr,
            *rt = nullptr;
+    SyncProg cg_eres, cg_db;  // the CG's part of the Eres (zero far field) and dB syncs
+    bool cg_syncs = false;
     int res_its = 0;
     double res_rel = 0.0;
     static constexpr int RES_CHECK = 4;  // the residual is read back every RES_CHECK iterations
@@ -1497,6 +1517,7 @@ public:
             caller_plan[gid] = true;
         }
         plan_h[gid][stage] = std::move(ent);
+        if (gid == G_ERES0 || gid == G_DB) cg_syncs = false;
         upload_plans(gid);
         build_all_merged();
         drop_graph();
@@ -1662,7 +1683,7 @@ public:
     static constexpr unsigned MG_PREPARE_PAIR = (1u << G_BADD) | (1u << G_BFACE);
 
     static constexpr int kPhaseHalo = 4, kPhaseOwner = 5;  // phases of a group's program (A, B, C, D, H, E)
-    std::vector<SyncPlan::Host> plan_group(SyncPlan &plan, int gid) {
+    std::vector<SyncPlan::Host> plan_group(SyncPlan &plan, int gid, const std::function<bool(int, int)> &keep = nullptr) {
         plan.out.clear();
         for (const GField &gf : group_fields(gid, nspecies())) {
             std::vector<const SyncOp *> ops;
@@ -1679,7 +1700,7 @@ public:
                             }
                     }
             }
-            plan.add(ops, gf.slot, gf.ncomp, F->blk[0].g);
+            plan.add(ops, gf.slot, gf.ncomp, F->blk[0].g, keep ? [&](int x) { return keep(x, gf.loc); } : std::function<bool(int)>());
         }
         return std::move(plan.out);
     }
@@ -1701,6 +1722,9 @@ public:
                                             reinterpret_cast<const int *>(p.mem.p + at[n][1]), p.mem.p + at[n][2]});
     }
 
+    void run_prog(const SyncProg &p, hipStream_t s) {
+        for (const SyncLaunch &l : p.launches) launch_sync(s, l.waves, l.nw, l.ent, l.val, Fd(), P);
+    }
     void run_merged(unsigned gset) { run_merged(gset, st); }
     void run_merged(unsigned gset, hipStream_t s) {
         auto it = mprog.find(gset);
@@ -1709,7 +1733,7 @@ public:
             upload_prog(mprog[gset], plan_group(plan, __builtin_ctz(gset)));
             it = mprog.find(gset);
         }
-        for (const SyncLaunch &l : it->second.launches) launch_sync(s, l.waves, l.nw, l.ent, l.val, Fd(), P);
+        run_prog(it->second, s);
         // caller plans: the halo stage of every group of the set, then the owner stage
         for (int t = 0; t < 2; ++t)
             for (int gid = 0; gid < G_NGROUP; ++gid)
@@ -1836,6 +1860,30 @@ public:
         rwd = v + 8 * m;
         r_part.upload(std::vector<double>(3 * (size_t)std::max(res_blocks(n), 1), 0.0));
         r_S.upload(std::vector<double>(CG_NSCALAR, 0.0));
+        // The CG's syncs write only what its curls read: of Eres the owned edges,
+        // of dB the owned faces and the first ghosts, within a point of the
+        // unknowns' range.  (A patch connection's plan may read ghosts of its own
+        // level, so there the whole sync runs.)
+        if (!caller_plan[G_ERES0] && !caller_plan[G_DB]) {
+            const std::vector<int> &lo = R_res.hlo, &nn = R_res.hn;
+            for (int gid : {G_ERES0, G_DB}) {
+                const bool face = gid == G_DB;
+                SyncPlan plan(F->Vtot);
+                auto keep = [&, face](int x, int loc) {
+                    int p[4], hi[3];
+                    F->point_of(x, p);
+                    F->owned_hi(p[0], loc, hi);
+                    for (int a = 0; a < 3; ++a) {
+                        const int l = lo[3 * p[0] + a], h = l + nn[3 * p[0] + a], i = p[1 + a];
+                        if (h == l || i < l - 1 || i > h) return false;
+                        if (face ? (i < -1 || i > F->blk[p[0]].m[a]) : (i < 0 || i >= hi[a])) return false;
+                    }
+                    return true;
+                };
+                upload_prog(face ? cg_db : cg_eres, plan_group(plan, gid, keep));
+            }
+            cg_syncs = true;
+        }
     }
 
     // MatMultImplicitResistive_ (Mercury_ImplicitResistive.cpp:406-465): Eres <- x on
@@ -1843,12 +1891,16 @@ public:
     // alpha * CurlAdjFaceToEdge(beta * dB), alias mean, y = Eres - eta * dJ.  The
     // reference's Sync(dJ) touches no unknown and is left out.  lin: the far-field
     // Eres handler with a zero field (the linear part).  With w, the partial sums of
-    // x.y.w go to r_part.  scattered: x is already in the Eres slots of the unknowns.
+    // x.y.w go to r_part.  scattered: x is already in the Eres slots of the
+    // unknowns (the iterations: their syncs leave out the ghosts that no curl reads).
     void res_apply(const double *x, double *y, double dt, bool lin, const double *w, bool scattered = false) {
         if (!scattered) launch_res_scatter(st, rd, x, Fd());
-        run_merged(1u << (lin ? G_ERES0 : G_ERES));
+        const bool part = scattered && cg_syncs;
+        if (part) run_prog(cg_eres, st);
+        else run_merged(1u << (lin ? G_ERES0 : G_ERES));
         launch_dec_d1(st, R_res.h, Bd(), Fd(), SL_ERES, SL_DB, -dt);
-        run_merged(1u << G_DB);
+        if (part) run_prog(cg_db, st);
+        else run_merged(1u << G_DB);
         launch_jedge(st, R_res.h, Bd(), Fd(), SL_DB, SL_DJ);
         alias.launch(st, Fd(), SL_DJ);
         singular_current(SL_DB, SL_DJ);
@@ -1897,6 +1949,7 @@ public:
             ++its;
         }
         res_its = its;
+        if (its > 0 && cg_syncs) run_merged(1u << G_DB);  // the rest of dB's ghosts, as the last application leaves them
         launch_res_scatter(st, rd, rx, Fd());
         run_merged(1u << G_ERES);
         launch_dec_d1(st, R_node.h, Bd(), Fd(), SL_ERES, SL_RHSBR, -1.0);

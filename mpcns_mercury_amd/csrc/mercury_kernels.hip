@@ -104,19 +104,18 @@ __global__ void k_jedge(const MercRange R, const MercBlk *__restrict__ B, double
     LOCATE(R);
     const MercBlk &bk = B[p.b];
     const long long q = p.q, di = OI(p), dj = OJ(p), dk = 1;
+    // the products that the three edges share are formed once, and nothing is
+    // stored before the last load (the slots may alias for the compiler); the
+    // edge past an upper face reads inside the box and is not stored
 #define BB(a, o) (F[SL_BETA + (a)][q + (o)] * F[sf + (a)][q + (o)])
-    if (p.i < bk.m[0]) {
-        const double v = (BB(1, -dk) - BB(1, 0)) + (BB(2, 0) - BB(2, -dj));
-        F[se + 0][q] = (1.0 * v) * F[SL_ALPHA + 0][q];
-    }
-    if (p.j < bk.m[1]) {
-        const double v = (BB(0, 0) - BB(0, -dk)) + (BB(2, -di) - BB(2, 0));
-        F[se + 1][q] = (1.0 * v) * F[SL_ALPHA + 1][q];
-    }
-    if (p.k < bk.m[2]) {
-        const double v = (BB(0, -dj) - BB(0, 0)) + (BB(1, 0) - BB(1, -di));
-        F[se + 2][q] = (1.0 * v) * F[SL_ALPHA + 2][q];
-    }
+    const double h0 = BB(0, 0), h1 = BB(1, 0), h2 = BB(2, 0);
+    const double v0 = (BB(1, -dk) - h1) + (h2 - BB(2, -dj));
+    const double v1 = (h0 - BB(0, -dk)) + (BB(2, -di) - h2);
+    const double v2 = (BB(0, -dj) - h0) + (h1 - BB(1, -di));
+    const double j0 = (1.0 * v0) * F[SL_ALPHA + 0][q], j1 = (1.0 * v1) * F[SL_ALPHA + 1][q], j2 = (1.0 * v2) * F[SL_ALPHA + 2][q];
+    if (p.i < bk.m[0]) F[se + 0][q] = j0;
+    if (p.j < bk.m[1]) F[se + 1][q] = j1;
+    if (p.k < bk.m[2]) F[se + 2][q] = j2;
 #undef BB
 }
 
@@ -760,12 +759,13 @@ __global__ void k_dec_d1(const MercRange R, const MercBlk *__restrict__ B, doubl
     LOCATE(R);
     const MercBlk &bk = B[p.b];
     const long long q = p.q, di = OI(p), dj = OJ(p), dk = 1;
-    if (p.j < bk.m[1] && p.k < bk.m[2])
-        F[s_face + 0][q] = mult * ((F[s_edge + 1][q] - F[s_edge + 1][q + dk]) + (F[s_edge + 2][q + dj] - F[s_edge + 2][q]));
-    if (p.i < bk.m[0] && p.k < bk.m[2])
-        F[s_face + 1][q] = mult * ((F[s_edge + 0][q + dk] - F[s_edge + 0][q]) + (F[s_edge + 2][q] - F[s_edge + 2][q + di]));
-    if (p.i < bk.m[0] && p.j < bk.m[1])
-        F[s_face + 2][q] = mult * ((F[s_edge + 0][q] - F[s_edge + 0][q + dj]) + (F[s_edge + 1][q + di] - F[s_edge + 1][q]));
+    // the nine edge values are read once, before the first store
+    const double e0 = F[s_edge + 0][q], e0j = F[s_edge + 0][q + dj], e0k = F[s_edge + 0][q + dk];
+    const double e1 = F[s_edge + 1][q], e1i = F[s_edge + 1][q + di], e1k = F[s_edge + 1][q + dk];
+    const double e2 = F[s_edge + 2][q], e2i = F[s_edge + 2][q + di], e2j = F[s_edge + 2][q + dj];
+    if (p.j < bk.m[1] && p.k < bk.m[2]) F[s_face + 0][q] = mult * ((e1 - e1k) + (e2j - e2));
+    if (p.i < bk.m[0] && p.k < bk.m[2]) F[s_face + 1][q] = mult * ((e0k - e0) + (e2 - e2i));
+    if (p.i < bk.m[0] && p.j < bk.m[1]) F[s_face + 2][q] = mult * ((e0 - e0j) + (e1i - e1));
 }
 // d2: face 2-form -> cell 3-form (outward flux sum), owned cells
 __global__ void k_dec_d2(const MercRange R, const MercBlk *__restrict__ B, double *const *__restrict__ F_, int s_face, int s_cell) {
