@@ -46,7 +46,10 @@ enum MercSlot {
     SL_NANEU = SL_PEN + 1,
     // the third ion species (He++): state, PV, RHS and step-start copy
     SL_UHE = SL_NANEU + 1, SL_PVHE = SL_UHE + 5, SL_RHE = SL_PVHE + 5, SL_U0HE = SL_RHE + 5,
-    SL_NSLOT = SL_U0HE + 5
+    // cell: the 3x3 inverse of the J reconstruction (row-major), whose products
+    // with the edge vectors around the cell are the 36 weights SL_WJ
+    SL_WJM = SL_U0HE + 5,
+    SL_NSLOT = SL_WJM + 9
 };
 
 // species order H+, Na+, He++ (the reference's two first: every sum over

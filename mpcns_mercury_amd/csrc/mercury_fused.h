@@ -28,9 +28,10 @@ void launch_to_double(hipStream_t st, const float *src, double *dst, long long n
 void launch_bcell_jedge(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, bool mix,
                         double *divb_part = nullptr, double *divb_mon = nullptr);
 void launch_divb_monitor_reset(hipStream_t st, double *divb_mon);
-// dt_next, when not null: also clears the dt words of the nruns runs
+// products: a device word, 1 while the J weights are products of SL_WJM and the
+// edge vectors.  dt_next, when not null: also clears the dt words of the nruns runs
 void launch_jcell_t(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, bool mix,
-                    unsigned long long *dt_next = nullptr, int nruns = 0);
+                    const int *products, unsigned long long *dt_next = nullptr, int nruns = 0);
 void launch_to_float(hipStream_t st, const double *src, float *dst, long long n);
 // per run: the abort rule on the smallest of its dt words, dt[r] committed, status 4 words per run
 void launch_dt_commit(hipStream_t st, unsigned long long *dt, const unsigned long long *dt_next, unsigned long long *status, int nruns);

@@ -1168,12 +1168,18 @@ __global__ void k_bcell_jedge(const MercRange R, const MercBlk *__restrict__ B, 
     if (divb_part) group_max2(dmx, bmx, divb_part);
 }
 
-// calc_Jcell (MercurySolver_Current.cpp:203-259), owned cells.  With dt_next it
-// also clears the nwords dt words that the derived pass behind it fills (a launch
+// calc_Jcell (MercurySolver_Current.cpp:203-259), owned cells.  In FP64, while
+// *products says that the 36 weights are the context's own, they are formed from
+// the cell's 3x3 inverse and the edge vectors (which four cells share), with the
+// roundings of the stored ones: 336 -> 192 bytes a cell, 195 -> 129 us on 2.53 M
+// cells (3.8 TB/s), 7.7 -> 5.4 on 48^3.  The mixed form's weights
+// are FP32 roundings of the products, which FP32 factors do not give.  With
+// dt_next it also clears the nwords dt words that the derived pass behind it fills (a launch
 // of their own costs a small step more than the clearing does).
 template <bool MIX>
 __global__ void k_jcell_t(const MercRange R, const MercBlk *__restrict__ B, double *const *__restrict__ F_,
-                          const float *const *__restrict__ G_, unsigned long long *__restrict__ dt_next, int nwords) {
+                          const float *const *__restrict__ G_, const int *__restrict__ products, unsigned long long *__restrict__ dt_next,
+                          int nwords) {
     if (dt_next)
         for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < nwords; t += gridDim.x * blockDim.x)
             dt_next[(long long)t * DT_LINE] = (unsigned long long)__double_as_longlong(1e100);
@@ -1186,10 +1192,26 @@ __global__ void k_jcell_t(const MercRange R, const MercBlk *__restrict__ B, doub
                      (T)F[SL_J + 1][q], (T)F[SL_J + 1][q + di], (T)F[SL_J + 1][q + 1], (T)F[SL_J + 1][q + di + 1],
                      (T)F[SL_J + 2][q], (T)F[SL_J + 2][q + di], (T)F[SL_J + 2][q + dj], (T)F[SL_J + 2][q + di + dj]};
     T J[3] = {T(0), T(0), T(0)};
+    bool own = false;
+    if constexpr (!MIX) own = *products != 0;
+    if (own) {
+        T M[9];
 #pragma unroll
-    for (int n = 0; n < 12; ++n)
+        for (int c = 0; c < 9; ++c) M[c] = F[SL_WJM + c][q];
+        const long long at[12] = {q, q + dj, q + 1, q + dj + 1, q, q + di, q + 1, q + di + 1, q, q + di, q + dj, q + di + dj};
 #pragma unroll
-        for (int c = 0; c < 3; ++c) J[c] += st<MIX>(F, G, SL_WJ + 12 * c + n, q) * s[n];
+        for (int n = 0; n < 12; ++n) {
+            const int a = n / 4;
+            const T l0 = F[SL_DR + 3 * a][at[n]], l1 = F[SL_DR + 3 * a + 1][at[n]], l2 = F[SL_DR + 3 * a + 2][at[n]];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) J[c] += (M[3 * c] * l0 + M[3 * c + 1] * l1 + M[3 * c + 2] * l2) * s[n];
+        }
+    } else {
+#pragma unroll
+        for (int n = 0; n < 12; ++n)
+#pragma unroll
+            for (int c = 0; c < 3; ++c) J[c] += st<MIX>(F, G, SL_WJ + 12 * c + n, q) * s[n];
+    }
     for (int c = 0; c < 3; ++c) F[SL_JC + c][q] = (double)J[c];
 }
 
@@ -1311,9 +1333,9 @@ void launch_divb_monitor_reset(hipStream_t st, double *divb_mon) {
     hipLaunchKernelGGL(k_divb_monitor_reset, dim3(1), dim3(64), 0, st, divb_mon);
 }
 void launch_jcell_t(hipStream_t st, const RangeH &R, const MercBlk *B, double *const *F, const float *const *G, bool mix,
-                    unsigned long long *dt_next, int nruns) {
-    if (mix) LAUNCH_R(k_jcell_t<true>, R, B, F, G, dt_next, nruns * DT_WORDS);
-    else LAUNCH_R(k_jcell_t<false>, R, B, F, G, dt_next, nruns * DT_WORDS);
+                    const int *products, unsigned long long *dt_next, int nruns) {
+    if (mix) LAUNCH_R(k_jcell_t<true>, R, B, F, G, products, dt_next, nruns * DT_WORDS);
+    else LAUNCH_R(k_jcell_t<false>, R, B, F, G, products, dt_next, nruns * DT_WORDS);
 }
 void launch_to_float(hipStream_t st, const double *src, float *dst, long long n) {
     if (n > 0) hipLaunchKernelGGL(k_to_float, dim3(nblk(n, 256)), dim3(256), 0, st, src, dst, n);

@@ -224,7 +224,8 @@ void BlockGeom::compute(const MercPhys &P, SlotWriter &out) {
 
     // reconstruction weights on owned cells
     {
-        std::vector<double> Wb[18], Wj[36];
+        std::vector<double> Wb[18], Wj[36], Wjm[9];
+        for (auto &v : Wjm) v.assign(V, 0.0);
         for (auto &v : Wb) v.assign(V, 0.0);
         for (auto &v : Wj) v.assign(V, 0.0);
         const double epsw = 1.0e-30, eig_tol = 1.0e-10;
@@ -319,12 +320,16 @@ void BlockGeom::compute(const MercPhys &P, SlotWriter &out) {
                         for (int a = 0; a < 3; ++a)
                             for (int c = 0; c < 3; ++c) Mi[a][c] += Vv[a][t] * inv * Vv[c][t];
                     }
+                    for (int a = 0; a < 3; ++a)
+                        for (int c = 0; c < 3; ++c) Wjm[3 * a + c][q] = Mi[a][c];
+                    for (int n = 0; n < 12; ++n) wj_products &= actj[n];
                     for (int n = 0; n < 12; ++n)
                         if (actj[n])
                             for (int a = 0; a < 3; ++a) Wj[12 * a + n][q] = Mi[a][0] * l[n][0] + Mi[a][1] * l[n][1] + Mi[a][2] * l[n][2];
                 }
         for (int c = 0; c < 18; ++c) out.put(SL_WB + c, Wb[c]);
         for (int c = 0; c < 36; ++c) out.put(SL_WJ + c, Wj[c]);
+        for (int c = 0; c < 9; ++c) out.put(SL_WJM + c, Wjm[c]);
     }
 
     // Hall taper and local artificial eta per owned edge

@@ -20,6 +20,7 @@ struct BlockGeom {
     long long V, Vn;
     std::array<std::vector<double>, 3> X;    // node coordinates, ghost depth g+1
     std::array<std::vector<double>, 9> JD_;  // face area vectors (kept for the initial face fluxes)
+    bool wj_products = true;  // every J weight is its cell's SL_WJM times the edge vector (no collapsed edge was left out)
 
     BlockGeom(const int m_[3], int g_, const double *owned_nodes);
     long long idx(int i, int j, int k) const { return ((long long)(i + g) * N[1] + (j + g)) * N[2] + (k + g); }

@@ -981,6 +981,18 @@ public:
     float **fptr = nullptr;                   // device table indexed like the FP64 slots (null where absent)
     std::vector<int> fslots;                  // FP32 static copies
     std::vector<int> islots;                  // FP32 derived intermediates of the mixed form
+    // device word: 1 while the J weights are products of SL_WJM and the edge vectors,
+    // 0 once a caller has written either or holds the address of one
+    DBuf<int> wj_products;
+    bool wj_own = false;
+    void static_written(int slot) {
+        const bool wj = slot >= SL_WJ && slot < SL_WJ + 36, dr = slot >= SL_DR && slot < SL_DR + 9;
+        if (!wj_own || !(wj || dr)) return;
+        const int no = 0;
+        HIPCHK(hipStreamSynchronize(st));
+        HIPCHK(hipMemcpy(wj_products.p, &no, sizeof(no), hipMemcpyHostToDevice));
+        wj_own = false;
+    }
     unsigned long long *d_red = nullptr;      // reduction result (2 words)
     double *d_part = nullptr;                 // per-workgroup partial maxima of the div B diagnostic
     // the div B monitor of the fused derived pass: per-workgroup maxima and
@@ -1122,6 +1134,9 @@ public:
             w.b = b;
             geom[b]->compute(Pb(b), w);
         }
+        wj_own = true;
+        for (const auto &q : geom) wj_own &= q->wj_products;
+        wj_products.upload(std::vector<int>(1, wj_own ? 1 : 0));
         // FP32 static copies: reconstruction weights, Hodge stars, edge geometry, taper, eta, photo rate
         for (int c = 0; c < 18; ++c) fslots.push_back(SL_WB + c);
         for (int c = 0; c < 36; ++c) fslots.push_back(SL_WJ + c);
@@ -1968,7 +1983,7 @@ public:
         alias.launch(st, Fd(), SL_J);
         singular_current(SL_B, SL_J);
         run_merged(MG_DERIVED_PAIR);
-        launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix(), final ? d_dt_next : nullptr, nruns);
+        launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix(), wj_products.p, final ? d_dt_next : nullptr, nruns);
         sync(G_JCELL);
         launch_cell_end(st, R_box.h, Bd(), Fd(), Gd(), P, d_dt_next, final ? 1 : 0, mix(), nruns);
     }
@@ -2000,7 +2015,7 @@ public:
         } else {
             run_merged(MG_DERIVED_PAIR, st);
         }
-        launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix(), final ? d_dt_next : nullptr, nruns);
+        launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix(), wj_products.p, final ? d_dt_next : nullptr, nruns);
         sync(G_JCELL);
         HIPCHK(hipEventRecord(ev_join2, st2));
         HIPCHK(hipStreamWaitEvent(st, ev_join2, 0));
@@ -2337,7 +2352,7 @@ public:
         else if (op == "update_all") launch_update_all(st, R_node.h, Bd(), Fd(), Gd(), dtp(), mix(), nspecies());
         else if (op == "bcell_jedge") launch_bcell_jedge(st, R_node.h, Bd(), Fd(), Gd(), mix());
         else if (op == "bcell_jedge_monitor") launch_bcell_jedge(st, R_node.h, Bd(), Fd(), Gd(), mix(), d_mpart, d_mon);
-        else if (op == "jcell_t") launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix());
+        else if (op == "jcell_t") launch_jcell_t(st, R_cell.h, Bd(), Fd(), Gd(), mix(), wj_products.p);
         else if (op == "sync_all") {
             for (int gid = 0; gid < G_NGROUP; ++gid) sync(gid);
         }
@@ -2629,6 +2644,7 @@ int mercury_field_device(MercuryContext *ctx, const char *name, int block, int c
         const int slot = field_comp_slot(name, comp);
         HIPCHK(hipStreamSynchronize(ctx->s->st));
         ctx->s->materialize(slot);
+        ctx->s->static_written(slot);
         *ptr = ctx->s->F->hptr[slot] + ctx->s->F->blk[block].off;
     })
 }
@@ -2672,6 +2688,7 @@ int mercury_set_sync_plan(MercuryContext *ctx, const char *group, int stage, lon
             ent.insert(ent.end(), {x[0], d, x[5], src, x[10]});
         }
         HIPCHK(hipStreamSynchronize(S.st));
+        for (size_t e = 0; e < ent.size(); e += 5) S.static_written(ent[e]);
         S.set_sync_plan(gid, stage, std::move(ent));
     })
 }
@@ -2771,7 +2788,9 @@ int mercury_upload(MercuryContext *ctx, const char *name, int block, int comp, c
     ABI_TRY({
         if (block < 0 || block >= ctx->s->F->nb() || !host) throw std::runtime_error("invalid block or buffer");
         HIPCHK(hipStreamSynchronize(ctx->s->st));
-        ctx->s->F->upload_block(field_comp_slot(name, comp), block, host);
+        const int slot = field_comp_slot(name, comp);
+        ctx->s->static_written(slot);
+        ctx->s->F->upload_block(slot, block, host);
     })
 }
 
