@@ -116,6 +116,35 @@ def test_dec_diagnostics_bit_exact(oracle_mod, dims, g):
             x.free()
 
 
+# a plane of 16 x 16 cells is one partial maximum: one, whole and odd numbers of
+# the folding group's 1024 threads and four loads each
+@pytest.mark.parametrize("groups", [1, 17, 1024, 1025, 4096, 4097, 9001])
+def test_dec_maximum_in_any_partial(oracle_mod, groups):
+    print(f"[case] DEC diagnostic of {groups} partial maxima", flush=True)
+    L = hip.load()
+    dims, g = (groups, 16, 16), 0
+    sh = orc._box_shape(dims, g)
+    rng = np.random.default_rng(groups)
+    edge = _rand(sh, rng, 3)
+    res = hipmem.DeviceArray(np.full(1, -1.0))
+    try:
+        for at in sorted({0, groups // 2, max(0, groups - 2)}):
+            e = [x.copy() for x in edge]
+            for x in e:
+                x[at, 7, 9] *= 1e3
+            de = [hipmem.DeviceArray(x) for x in e]
+            try:
+                for call in (L.mercury_dec_max_abs_div_curl, L.mercury_dec_max_abs_div_curl_noalloc):
+                    _chk(call(_dims(dims), g, hipmem.ptrs(de), res.ptr, None))
+                    hipmem.synchronize()
+                    assert res.download()[0] == orc.dec_max_abs_div_curl(dims, g, e)
+            finally:
+                for x in de:
+                    x.free()
+    finally:
+        res.free()
+
+
 def test_dec_invalid_arguments_fail_with_a_message():
     """Bad sizes and NULL arrays are refused before anything is launched."""
     L = hip.load()
