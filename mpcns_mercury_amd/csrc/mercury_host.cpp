@@ -330,6 +330,135 @@ struct SyncProg {
     std::vector<SyncLaunch> launches;
 };
 
+// Plans applied one after the other (each: entries (dst slot, dst, src slot, src,
+// sign), every read before every write; of two entries with one destination the
+// later one stands) as one launch: an entry whose source an earlier plan writes
+// takes that plan's source, and a replaced entry is left out.  Copies that read
+// what others write go into one wave, which loads before it stores: the chains of
+// patch connections are two to four entries long.
+class PlanJoin {
+public:
+    explicit PlanJoin(long long nvalues) : words((size_t)(nvalues + 63) / 64) {}
+    void add(const std::vector<int> &plan) {
+        const size_t first = all.size();
+        std::vector<size_t> need;  // entries that read what an earlier plan writes
+        Marks needed(words), twice(words);
+        for (size_t q = 0; q + 4 < plan.size(); q += 5) {
+            const Entry e{plan[q], plan[q + 1], plan[q + 2], plan[q + 3], plan[q + 4]};
+            if (dst.get(e.ss, e.s)) {
+                need.push_back(all.size());
+                needed.set(e.ss, e.s);
+            }
+            all.push_back(e);
+        }
+        if (!need.empty()) {
+            std::vector<std::pair<std::pair<int, int>, size_t>> by;
+            for (size_t i = 0; i < first; ++i)
+                if (needed.get(all[i].ds, all[i].d)) by.push_back({{all[i].ds, all[i].d}, i});
+            std::sort(by.begin(), by.end());
+            for (size_t n : need) {
+                Entry &e = all[n];
+                const Entry &w = all[std::lower_bound(by.begin(), by.end(), std::make_pair(std::make_pair(e.ss, e.s), (size_t)0))->second];
+                e = {e.ds, e.d, w.ss, w.s, e.sign * w.sign};
+            }
+        }
+        bool any = false;
+        for (size_t i = first; i < all.size(); ++i)
+            if (dst.set(all[i].ds, all[i].d)) any = twice.set(all[i].ds, all[i].d) || true;
+        if (!any) return;
+        Marks seen(words);
+        size_t keep = all.size();
+        for (size_t i = all.size(); i-- > 0;)
+            if (!twice.get(all[i].ds, all[i].d) || !seen.set(all[i].ds, all[i].d)) all[--keep] = all[i];
+        all.erase(all.begin(), all.begin() + keep);
+    }
+    // entries (dst, src, dst slot | src slot << 16, sign * number of components from
+    // those slots on), 64 of one number a wave, padded with dst -1; false: a chain
+    // does not fit a wave
+    bool emit(std::vector<int> &out) const {
+        Marks src(words);
+        for (const Entry &e : all) src.set(e.ss, e.s);
+        // by number of components and slot: a wave's lanes mostly share theirs
+        std::vector<std::vector<size_t>> plain[kRun + 1];
+        for (auto &v : plain) v.resize(SL_NSLOT);
+        std::vector<size_t> linked;
+        auto is_linked = [&](const Entry &e) { return dst.get(e.ss, e.s) || src.get(e.ds, e.d); };
+        for (size_t i = 0, n; i < all.size(); i += n) {
+            n = 1;
+            if (is_linked(all[i])) {
+                linked.push_back(i);
+                continue;
+            }
+            auto next = [&](const Entry &a, const Entry &b) {
+                return b.d == a.d && b.s == a.s && b.sign == a.sign && b.ds == a.ds + 1 && b.ss == a.ss + 1;
+            };
+            while (n < kRun && i + n < all.size() && next(all[i + n - 1], all[i + n]) && !is_linked(all[i + n])) ++n;
+            plain[n][all[i].ds].push_back(i);
+        }
+        auto put = [&](const Entry &e, int n) { out.insert(out.end(), {e.d, e.s, e.ds | e.ss << 16, e.sign * n}); };
+        auto fill_wave = [&] {
+            while (out.size() % 256) out.insert(out.end(), {-1, -1, 0, 1});
+        };
+        for (size_t n = 1; n <= kRun; ++n) {
+            for (const auto &v : plain[n])
+                for (size_t i : v) put(all[i], (int)n);
+            fill_wave();
+        }
+        const size_t n = linked.size();
+        auto key = [&](size_t a) { return std::make_pair(all[a].ds, all[a].d); };
+        std::sort(linked.begin(), linked.end(), [&](size_t a, size_t b) { return key(a) < key(b); });
+        std::vector<size_t> root(n), order(n);
+        for (size_t i = 0; i < n; ++i) root[i] = order[i] = i;
+        auto find = [&](size_t x) {
+            while (root[x] != x) x = root[x] = root[root[x]];
+            return x;
+        };
+        for (size_t i = 0; i < n; ++i) {
+            const Entry &e = all[linked[i]];
+            if (!dst.get(e.ss, e.s)) continue;
+            const size_t w = std::lower_bound(linked.begin(), linked.end(), std::make_pair(e.ss, e.s),
+                                              [&](size_t a, const std::pair<int, int> &k) { return key(a) < k; }) - linked.begin();
+            root[find(i)] = find(w);
+        }
+        for (size_t i = 0; i < n; ++i) root[i] = find(i);
+        std::sort(order.begin(), order.end(), [&](size_t a, size_t b) { return std::make_pair(root[a], a) < std::make_pair(root[b], b); });
+        for (size_t t = 0, u; t < n; t = u) {
+            for (u = t + 1; u < n && root[order[u]] == root[order[t]];) ++u;
+            if (u - t > 64) return false;
+            if (out.size() / 4 % 64 + (u - t) > 64) fill_wave();
+            for (size_t i = t; i < u; ++i) put(all[linked[order[i]]], 1);
+        }
+        fill_wave();
+        return true;
+    }
+
+private:
+    static constexpr size_t kRun = 5;
+    struct Entry {
+        int ds, d, ss, s, sign;
+    };
+    struct Marks {
+        explicit Marks(size_t w) : words(w), m(SL_NSLOT) {}
+        size_t words;
+        std::vector<std::vector<uint64_t>> m;  // a bit per value of the slots in use
+        bool get(int slot, int i) const { return !m[slot].empty() && (m[slot][i >> 6] >> (i & 63) & 1); }
+        bool set(int slot, int i) {  // whether it was set before
+            if (m[slot].empty()) m[slot].resize(words);
+            uint64_t &w = m[slot][i >> 6], b = (uint64_t)1 << (i & 63);
+            const bool was = w & b;
+            w |= b;
+            return was;
+        }
+    };
+    size_t words;
+    std::vector<Entry> all;
+    Marks dst{words};
+};
+struct PlanProg {
+    DBuf<int> ent;  // empty and !joined: the plans run stage by stage
+    bool joined = false;
+};
+
 // Turns the phases of a field's sync into as few launches as can be.  It follows
 // the ops in order, symbolically: what each value is after them, in terms of the
 // values before the first: a copy of one, a constant, or a wall state made of the
@@ -932,9 +1061,10 @@ public:
     // (dst slot, dst, src slot, src, sign) on arena indices
     bool caller_plan[G_NGROUP] = {};
     std::vector<int> plan_h[G_NGROUP][2];
+    std::map<unsigned, PlanProg> pprog;  // the plans of a set of groups, as mprog
+    // plans that do not join run stage by stage; one whose sources include its own
+    // destinations runs staged (every read before every write) through plan_tmp
     DBuf<int> plan_d[G_NGROUP][2];
-    // a plan whose sources include its own destinations runs staged (every
-    // read before every write) through plan_tmp
     bool plan_staged[G_NGROUP][2] = {};
     DBuf<double> plan_tmp[G_NGROUP][2];
     // patch connections (rotated, mirrored, partial-face interfaces): their
@@ -1480,6 +1610,7 @@ public:
         }
         build_all_merged();
     }
+    bool synced_group(int gid) const { return P.resist_enabled != 0.0 || (gid != G_ERES && gid != G_ERES0 && gid != G_DB); }
     // The sync programs of the groups and of the pairs that the step syncs
     // together.  The groups of the resistive correction are left to their first
     // use where there is no correction.
@@ -1487,7 +1618,7 @@ public:
         mprog.clear();
         std::vector<int> todo;
         for (int gid = 0; gid < G_NGROUP; ++gid)
-            if (P.resist_enabled != 0.0 || (gid != G_ERES && gid != G_ERES0 && gid != G_DB)) todo.push_back(gid);
+            if (synced_group(gid)) todo.push_back(gid);
         // the groups are independent: a few threads, each with a table of its own
         std::vector<SyncPlan::Host> h[G_NGROUP];
         std::atomic<size_t> next{0};
@@ -1534,9 +1665,44 @@ public:
         }
         plan_h[gid][stage] = std::move(ent);
         if (gid == G_ERES0 || gid == G_DB) cg_syncs = false;
-        upload_plans(gid);
         build_all_merged();
+        build_plans(1u << gid);
         drop_graph();
+    }
+    // The plans of the sets that a group of changed is in: the groups by themselves
+    // and the pairs that the step syncs together
+    void build_plans(unsigned changed) {
+        std::vector<unsigned> sets;
+        for (int gid = 0; gid < G_NGROUP; ++gid)
+            if (synced_group(gid)) sets.push_back(1u << gid);
+        for (unsigned pair : {MG_EDGE_PAIR, MG_STATE_PAIR, MG_DERIVED_PAIR, MG_PREPARE_PAIR}) sets.push_back(pair);
+        sets.erase(std::remove_if(sets.begin(), sets.end(), [&](unsigned s) { return !(s & changed); }), sets.end());
+        std::vector<std::vector<int>> ent(sets.size());
+        std::vector<char> joined(sets.size());
+        std::atomic<size_t> next{0};
+        auto work = [&] {
+            for (size_t t; (t = next++) < sets.size();) joined[t] = join_plans(sets[t], ent[t]);
+        };
+        std::vector<std::future<void>> pool;
+        if (F->Vtot > 100000)
+            for (int t = 0; t < 3; ++t) pool.push_back(std::async(std::launch::async, work));
+        work();
+        for (auto &f : pool) f.get();
+        for (size_t t = 0; t < sets.size(); ++t) upload_join(sets[t], joined[t], ent[t]);
+    }
+    bool join_plans(unsigned gset, std::vector<int> &ent) const {
+        PlanJoin J(F->Vtot);
+        for (int t = 0; t < 2; ++t)
+            for (int gid = 0; gid < G_NGROUP; ++gid)
+                if ((gset & (1u << gid)) && caller_plan[gid]) J.add(plan_h[gid][t]);
+        return J.emit(ent);
+    }
+    void upload_join(unsigned gset, bool joined, const std::vector<int> &ent) {
+        PlanProg &p = pprog[gset];
+        p.joined = joined;
+        p.ent.upload(joined ? ent : std::vector<int>());
+        for (int gid = 0; gid < G_NGROUP && !joined; ++gid)
+            if ((gset & (1u << gid)) && caller_plan[gid]) upload_plans(gid);
     }
     void upload_plans(int gid) {
         for (int t = 0; t < 2; ++t) {
@@ -1576,7 +1742,6 @@ public:
                 plan_h[gid][t] = std::move(out);
             }
             caller_plan[gid] = true;
-            upload_plans(gid);
         }
         const patch::EdgeClasses E = patch::edge_classes(T);
         std::vector<int> st{0}, mem, ms, max, ow, os, oax;
@@ -1595,6 +1760,7 @@ public:
         }
         alias.set(std::move(st), std::move(mem), std::move(ms), std::move(max), std::move(ow), std::move(os), std::move(oax));
         build_all_merged();
+        build_plans(~0u);
         // a singular edge has three or more aliases: without such a class there
         // is no registry to build (and no geometry to download)
         bool candidates = false;
@@ -1747,9 +1913,20 @@ public:
         if (it == mprog.end()) {  // a group of the resistive correction, by name, without the correction
             SyncPlan plan(F->Vtot);
             upload_prog(mprog[gset], plan_group(plan, __builtin_ctz(gset)));
+            if (caller_plan[__builtin_ctz(gset)]) {
+                std::vector<int> ent;
+                const bool joined = join_plans(gset, ent);
+                upload_join(gset, joined, ent);
+            }
             it = mprog.find(gset);
         }
         run_prog(it->second, s);
+        const auto pl = pprog.find(gset);
+        if (pl == pprog.end()) return;
+        if (pl->second.joined) {
+            launch_plan(s, pl->second.ent.p, pl->second.ent.n / 4, Fd());
+            return;
+        }
         // caller plans: the halo stage of every group of the set, then the owner stage
         for (int t = 0; t < 2; ++t)
             for (int gid = 0; gid < G_NGROUP; ++gid)

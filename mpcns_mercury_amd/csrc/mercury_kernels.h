@@ -48,6 +48,10 @@ void launch_alias_emf(hipStream_t st, const int *cls_start, const int *member, c
                       long long ncls, double *const *F);
 // one launch of a sync program: nw waves of 64 entries (ent: dst, src per entry)
 void launch_sync(hipStream_t st, const SyncWave *waves, long long nw, const int *ent, const double *val, double *const *F, const MercPhys &P);
+// n entries (dst, src, dst slot | src slot << 16, sign * components), whole waves of
+// 64 with one number of components, 1 to 5 (dst -1: none): dst <- sign * src, every
+// read of a wave before its writes
+void launch_plan(hipStream_t st, const int *ent, long long n, double *const *F);
 // n entries (dst slot, dst, src slot, src, sign): dst <- sign * src
 void launch_copy_plan(hipStream_t st, const int *ent, long long n, double *const *F);
 // the same entries with every read before every write (sources that are also

@@ -112,3 +112,75 @@ def test_plan_entry_semantics_and_refusals():
             g.set_sync_plan("Bfaces", 0, [])
     finally:
         g.close()
+
+
+# every length that a joined plan can hold in a wave, one more, and one that spans workgroups
+@pytest.mark.parametrize("lengths", [(1, 2, 3, 4, 5), (63, 1, 62, 2, 64), (65,), (300, 2, 64)])
+def test_joined_plans_read_before_they_write(lengths):
+    """Random plans of both stages on the groups of a pair, with chains (an entry
+    reads what the next one writes), cycles, signs, components and blocks mixed, and
+    owner entries that read and replace what the halo stage wrote: each plan acts as
+    one gather and one scatter, in the order halo stages, owner stages.  Bit for bit
+    (copies and sign flips)."""
+    case = _external(cases.make_split_cube(n=(12, 12, 10), split=(2, 1, 1)))
+    print(f"[case] joined plans, chains of {lengths}", flush=True)
+    rng = np.random.default_rng(sum(lengths))
+    box, gg = case.box(0), case.g
+    groups = {"Ucell": [("U_H", c) for c in range(5)] + [("U_Na", c) for c in range(5)], "Bface": [(f"B_{a}", 0) for a in ("xi", "eta", "zeta")]}
+    start = {n: rng.standard_normal((case.nb, field_info(n)[1]) + box) for n in {n for v in groups.values() for n, _ in v}}
+
+    def point(name, c):
+        # owned cells of both blocks, faces with them
+        return (name, c, int(rng.integers(case.nb))) + tuple(int(rng.integers(0, m - 2 * gg - 1)) for m in box)
+
+    def row(d, s, sign):
+        return [field_info(d[0])[0] + d[1], *d[2:], field_info(s[0])[0] + s[1], *s[2:], sign]
+
+    plans = {}
+    for grp, comps in groups.items():
+        pick = lambda: point(*comps[int(rng.integers(len(comps)))])  # noqa: E731
+        seen, halo = set(), []
+
+        def fresh():
+            p = pick()
+            while p in seen:
+                p = pick()
+            seen.add(p)
+            return p
+
+        for n in lengths:
+            pts = [fresh() for _ in range(n + 1)]
+            if n > 2 and n % 2:
+                pts[n] = pts[0]  # a cycle
+            halo += [(pts[i], pts[i + 1], int(rng.choice([-1, 1]))) for i in range(n)]
+        halo += [(fresh(), fresh(), 1) for _ in range(150)]
+        halo = [halo[i] for i in rng.permutation(len(halo))]
+        # an owner entry replaces a halo value, reads one, or neither
+        owner = [(halo[i][0], fresh(), -1) for i in range(0, 20)] + [(fresh(), halo[i][0], -1) for i in range(20, 40)]
+        owner += [(halo[i][0], halo[i + 20][0], 1) for i in range(40, 60)] + [(fresh(), fresh(), -1) for _ in range(70)]
+        plans[grp] = (halo, owner)
+
+    def run(with_plans):
+        g = Mercury(case)
+        try:
+            for grp, stages in plans.items():
+                for t in (0, 1):
+                    g.set_sync_plan(grp, t, [row(*e) for e in stages[t]] if with_plans else np.zeros((0, 11), np.int32))
+            for n, v in start.items():
+                for ib in range(case.nb):
+                    g.set(n, ib, v[ib])
+            g.op("sync_ucell")
+            g.op("sync_bface")
+            return {n: np.stack([g.get(n, ib) for ib in range(case.nb)]) for n in start}
+        finally:
+            g.close()
+
+    want, got = run(False), run(True)
+    at = lambda p: (p[2], p[1], p[3] + gg, p[4] + gg, p[5] + gg)  # noqa: E731
+    for stages in plans.values():
+        for plan in stages:
+            vals = [sign * want[s[0]][at(s)] for _, s, sign in plan]
+            for (d, _, _), v in zip(plan, vals):
+                want[d[0]][at(d)] = v
+    for n in start:
+        np.testing.assert_array_equal(got[n], want[n], err_msg=n)
