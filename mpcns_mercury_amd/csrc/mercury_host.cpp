@@ -2136,9 +2136,8 @@ public:
             // p is in the Eres slots already (scattered by the init or by the
             // previous iteration's k_cg_pxs)
             res_apply(rp, rAp, dt, true, rw, true);
-            launch_cg_pap(st, n, r_part.p, r_S.p);
-            launch_cg_r(st, n, r_S.p, rAp, rwd, rr, r_part.p, r_S.p);
-            launch_cg_pxs(st, rd, r_S.p, rr, rdg, rp, rx, Fd());
+            launch_cg_r(st, n, its, r_S.p, rAp, rwd, rr, r_part.p);
+            launch_cg_pxs(st, rd, its, r_S.p, r_part.p, rr, rdg, rp, rx, Fd());
             ++its;
         }
         res_its = its;
