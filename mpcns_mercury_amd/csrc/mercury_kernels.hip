@@ -608,7 +608,7 @@ __global__ void k_rk2(const MercRange R, const MercBlk *__restrict__ B, double *
 // A sync (halo, physical boundaries, owner -> alias) is one launch: the host
 // follows the reference's phases symbolically and leaves, for every value that
 // the sync changes, where it comes from among the values before the sync (see
-// SyncPlan in mercury_host.cpp).  Every wave has one kind of entry and one field,
+// SyncPlan in mercury_sync_plan.h).  Every wave has one kind of entry and one field,
 // so its slots and their pointers are scalar, and a lane reads all components of
 // its source before it writes one: one memory latency per entry.  Bound by launch
 // latency on small blocks (one launch in place of two to five, 7.0 -> 3.6 us per
