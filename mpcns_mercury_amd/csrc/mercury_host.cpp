@@ -1273,7 +1273,7 @@ public:
             };
             for (const GField &gf : group_fields(gid, nspecies())) {
                 const auto sl = slots_of(gf);
-                std::vector<int> fillA, copyB, setd, wallC, zeroC, copyD, haloH, ownE;
+                std::vector<int> fillA, copyB, setd, wallC[6], zeroC, copyD, haloH, ownE;
                 std::vector<double> setv;
                 const double *fill = nullptr;
                 static const double zero3[3] = {0, 0, 0};
@@ -1340,14 +1340,14 @@ public:
                             auto cl = [&](int v, int a) { return std::min(std::max(v, lo[a]), hi[a] - 1); };
                             for_box(inner_slab(Fl, b, LOC_CELL, dir), [&](int i, int j, int kk) {
                                 int c[3] = {i, j, kk};
-                                wallC.push_back(Fl.gidx(b, i, j, kk));
+                                wallC[f].push_back(Fl.gidx(b, i, j, kk));
                                 int r[3] = {c[0], c[1], c[2]};
                                 r[ax] -= sgn;
-                                wallC.push_back(Fl.gidx(b, cl(r[0], 0), cl(r[1], 1), cl(r[2], 2)));
+                                wallC[f].push_back(Fl.gidx(b, cl(r[0], 0), cl(r[1], 1), cl(r[2], 2)));
                                 for (int l = 1; l <= k.g; ++l) {
                                     int q[3] = {c[0], c[1], c[2]};
                                     q[ax] += l * sgn;
-                                    wallC.push_back(Fl.gidx(b, cl(q[0], 0), cl(q[1], 1), cl(q[2], 2)));
+                                    wallC[f].push_back(Fl.gidx(b, cl(q[0], 0), cl(q[1], 1), cl(q[2], 2)));
                                 }
                             });
                         } else if (gf.kind == K_JCELL) {
@@ -1371,8 +1371,10 @@ public:
                 if (!setd.empty()) add(A, OP_SETV, sl, std::move(setd), std::move(setv));
                 add(Bc, OP_COPY, sl, std::move(copyB));
                 const double na_floor[5] = {P.wall_rho_floor_Na, 0.0, 0.0, 0.0, P.wall_p_floor / (P.gamma - 1.0)};
-                if (!wallC.empty())
-                    add(C, OP_WALLF, sl, std::move(wallC), {}, gf.kind == K_UNA ? na_floor : nullptr, gf.kind == K_UNA ? 1 : (gf.kind == K_UHE ? 2 : 0));
+                // one op per face, in the order of the faces: where two walls meet, or
+                // stand two cells apart, the later one reads what the earlier one sets
+                for (auto &w : wallC)
+                    add(C, OP_WALLF, sl, std::move(w), {}, gf.kind == K_UNA ? na_floor : nullptr, gf.kind == K_UNA ? 1 : (gf.kind == K_UHE ? 2 : 0));
                 if (!zeroC.empty()) {
                     static const double z[10] = {0};
                     add(C, OP_FILL, sl, std::move(zeroC), {}, z);

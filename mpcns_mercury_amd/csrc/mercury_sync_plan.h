@@ -55,8 +55,11 @@ public:
         size_t at = 0, launch = 0;
         for (size_t u = 0; u < ends.size();) {
             size_t last = ends.size() - 1;
-            // one op by itself always can: no destination of it is a source of it
-            while (!(follow(ops, at, ends[last], slot, ncomp, g) && (last + 1 < ends.size() || !keep || drop(keep)) && joins()) && last > u) --last;
+            while (!(follow(ops, at, ends[last], slot, ncomp, g) && (last + 1 < ends.size() || !keep || drop(keep)) && joins())) {
+                // an op by itself can: no destination of it is a source of it
+                if (last == u) throw std::logic_error("sync plan: an op reads what it sets");
+                --last;
+            }
             emit(launch++, slot, ncomp);
             at = ends[last];
             u = last + 1;

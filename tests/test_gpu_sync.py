@@ -82,3 +82,74 @@ def test_ensemble_syncs_like_its_runs():
         base += c.nb
         m.close()
     e.close()
+
+
+def _walled(faces, blocks=((7, 6, 5), (5, 8, 6)), he=False):
+    """The shell's sectors with solid surfaces on the listed faces of each block."""
+    case = cases.make_shell(blocks=blocks, he=he)
+    for b, on in zip(case.blocks, faces):
+        b.bc = tuple(cases.BC_WALL if f in on else cases.BC_FARFIELD for f in range(6))
+    return case
+
+
+def _thin(case, n):
+    """Block 0 cut to its first n cells along the first axis."""
+    b, end = case.blocks[0], n + 1 + 2 * case.g
+    b.dims, b.nodes = (n,) + tuple(b.dims[1:]), np.ascontiguousarray(b.nodes[:, :n + 1])
+    case.fields[0] = {k: np.ascontiguousarray(v[:, :end]) for k, v in case.fields[0].items()}
+    return case
+
+
+WALLS = {
+    "adjacent": lambda he: _walled([(0, 2), (0,)], he=he),
+    "adjacent_upper": lambda he: _walled([(3, 5), (1,)], he=he),
+    "three": lambda he: _walled([(0, 3, 4), ()], he=he),
+    "six": lambda he: _walled([range(6), (2, 4)], he=he),
+    "opposite": lambda he: _walled([(0, 1), (0,)], he=he),
+    "two_cells_apart": lambda he: _thin(_walled([(0, 1), (0,)], he=he), 2),
+    "three_cells_apart": lambda he: _thin(_walled([(0, 1, 2), (0,)], he=he), 3),
+    # walls that meet, on blocks glued along the line where they do
+    "cut": lambda he: cases.split_block_case(_walled([(0, 2)], blocks=((12, 9, 10),), he=he), ((12,), (4, 5), (4, 6))),
+}
+
+
+@pytest.mark.parametrize("he", [False, True])
+@pytest.mark.parametrize("walls", list(WALLS))
+def test_sync_where_walls_meet(oracle_mod, walls, he):
+    """The wall states of random values, face after face: a later face reads what an
+    earlier one has set, and the blocks behind such a block get theirs too."""
+    case = WALLS[walls](he)
+    print(f"[case] walls {walls} he={he} dims={[b.dims for b in case.blocks]}", flush=True)
+    rng = np.random.default_rng(8)
+    g = Mercury(case)
+    o = oracle_mod.Oracle(case)
+    try:
+        names = ["U_H", "U_Na", "J_cell"] + (["U_He"] if he else [])
+        for name in names:
+            for ib in range(case.nb):
+                v = rng.uniform(0.1, 2.0, (field_info(name)[1],) + case.box(ib))
+                g.set(name, ib, v)
+                o.set(name, ib, v)
+        for op in ("sync_ucell", "sync_jcell"):
+            g.op(op)
+            o.op(op, 0)
+        for name in names:
+            for ib in range(case.nb):
+                np.testing.assert_array_equal(g.get(name, ib), o.get(name, ib), err_msg=f"{name}[{ib}]")
+    finally:
+        g.close()
+
+
+def test_steps_between_walls_that_meet(oracle_mod):
+    case = WALLS["adjacent"](False)
+    g = Mercury(case)
+    o = oracle_mod.Oracle(case)
+    try:
+        g.prepare()
+        o.prepare()
+        np.testing.assert_array_equal(g.step(2), o.step(2))
+        for name in ("U_H", "U_Na", "B_xi", "B_eta", "B_zeta", "J_cell"):
+            for ib in range(case.nb):
+                np.testing.assert_array_equal(g.get(name, ib), o.get(name, ib), err_msg=f"{name}[{ib}]")
+    finally:
+        g.close()
