@@ -905,6 +905,11 @@ public:
         HIPCHK(hipMemcpy(wj_products.p, &no, sizeof(no), hipMemcpyHostToDevice));
         wj_own = false;
     }
+    // a caller's values (upload, restart file) into one block's slot
+    void write_block(int slot, int b, const double *h) {
+        static_written(slot);
+        F->upload_block(slot, b, h);
+    }
     unsigned long long *d_red = nullptr;      // reduction result (2 words)
     double *d_part = nullptr;                 // per-workgroup partial maxima of the div B diagnostic
     // the div B monitor of the fused derived pass: per-workgroup maxima and
@@ -2748,9 +2753,7 @@ int mercury_upload(MercuryContext *ctx, const char *name, int block, int comp, c
     ABI_TRY({
         if (block < 0 || block >= ctx->s->F->nb() || !host) throw std::runtime_error("invalid block or buffer");
         HIPCHK(hipStreamSynchronize(ctx->s->st));
-        const int slot = field_comp_slot(name, comp);
-        ctx->s->static_written(slot);
-        ctx->s->F->upload_block(slot, block, host);
+        ctx->s->write_block(field_comp_slot(name, comp), block, host);
     })
 }
 
@@ -2889,7 +2892,7 @@ int mercury_read_restart(MercuryContext *ctx, const char *path, int *step, doubl
             for (int b = 0; b < F.nb(); ++b)
                 if (!kv.second[b])
                     throw std::runtime_error("restart: block " + std::to_string(b) + " of " + kv.first + " is inactive in the file");
-        for (const auto &kv : staged) F.upload_block(kv.first.first, kv.first.second, kv.second.data());
+        for (const auto &kv : staged) ctx->s->write_block(kv.first.first, kv.first.second, kv.second.data());
     })
 }
 

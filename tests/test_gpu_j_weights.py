@@ -6,6 +6,8 @@ import pytest
 from mpcns_mercury_amd import cases
 from mpcns_mercury_amd.hip import Mercury
 
+import restart_format as rf
+
 pytestmark = pytest.mark.gpu
 
 
@@ -54,4 +56,30 @@ def test_written_weights_are_used(field, how):
         a, own = _jcell(g), Ellipsis
     g.op("jcell")
     np.testing.assert_array_equal(a[1][own], g.get("J_cell", 1)[own])
+    g.close()
+
+
+@pytest.mark.parametrize("field", ["Jcell_from_Jedge_w", "dr_eta"])
+def test_weights_of_a_restart_file_are_used(tmp_path, field):
+    """A restart file may hold any field of the catalogue; weights or edge vectors
+    that it brings are the caller's, as uploaded ones are."""
+    g = Mercury(_case())
+    g.prepare()
+    g.step(2)  # J starts at zero
+    loc = rf.LOC_CODE["cell" if field[0] == "J" else "ey"]
+    blocks = []
+    for ib in range(g.case.nb):
+        hi = [m + 1 - d + g.case.g for m, d in zip(g.case.blocks[ib].dims, rf.DELTA_OF_CODE[loc])]
+        w = g.get(field, ib)[(slice(None),) + tuple(slice(0, h + g.case.g) for h in hi)]
+        blocks.append(((-g.case.g,) * 3, hi, 1.25 * w))
+    p = tmp_path / "weights.bin"
+    rf.write_restart(p, 0, 0.0, g.case.nb, [(field, loc, blocks[0][2].shape[0], g.case.g, blocks)])
+    before = _jcell(g)
+    g.read_restart(p)
+    a = _jcell(g)
+    g.op("jcell")
+    for ib in range(g.case.nb):
+        np.testing.assert_array_equal(a[ib], g.get("J_cell", ib))
+    if field[0] == "J":
+        assert any((x != y).any() for x, y in zip(a, before))
     g.close()
