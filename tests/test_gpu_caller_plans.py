@@ -184,3 +184,43 @@ def test_joined_plans_read_before_they_write(lengths):
                 want[d[0]][at(d)] = v
     for n in start:
         np.testing.assert_array_equal(got[n], want[n], err_msg=n)
+
+
+def test_plans_set_one_by_one_and_again():
+    """Each call plans only what it changes: plans set stage by stage with syncs in
+    between, replaced, and set in another order leave every group's sync (those of
+    the resistive correction, which this context has no program for at first, among
+    them) as a context that gets the last plans only."""
+    a = cases.make_split_cube(n=(12, 10, 8), split=(2, 2, 1), hall=True)
+    b = _external(a)
+    print("[case] caller plans one by one", flush=True)
+    ops = {"Ucell": "sync_ucell", "Bface": "sync_bface", "Eedge": "sync_eedge", "Ehall": "sync_ehall", "Jedge": "sync_jedge",
+           "B_cell": "sync_bcell", "J_cell": "sync_jcell", "Badd": "sync_badd", "Eres": "sync_eres", "dB": "sync_db"}
+    ga, gb, gc = Mercury(a), Mercury(b), Mercury(b)
+    try:
+        plans = {(grp, t): ga.sync_plan(grp, t) for grp in ops for t in (0, 1)}
+        for k, p in plans.items():
+            gc.set_sync_plan(*k, p)
+        rng = np.random.default_rng(4)
+        for n, (grp, t) in enumerate(sorted(plans, key=lambda k: (-k[1], k[0]))):
+            gb.set_sync_plan(grp, t, plans[grp, t][::3])
+            for op in list(ops.values())[n % 5::5]:
+                gb.op(op)
+        for k in reversed(plans):
+            gb.set_sync_plan(*k, plans[k])
+        names = INPUTS + ["E_xi", "E_eta", "E_zeta", "Ehall_xi", "Ehall_eta", "Ehall_zeta", "J_xi", "J_eta", "J_zeta", "B_cell", "J_cell",
+                          "Eres_xi", "Eres_eta", "Eres_zeta", "dB_xi", "dB_eta", "dB_zeta"]
+        for n in names:
+            for ib in range(b.nb):
+                v = rng.uniform(0.1, 2.0, (field_info(n)[1],) + b.box(ib))
+                gb.set(n, ib, v)
+                gc.set(n, ib, v)
+        for op in ops.values():
+            gb.op(op)
+            gc.op(op)
+        for n in names:
+            for ib in range(b.nb):
+                np.testing.assert_array_equal(gb.get(n, ib), gc.get(n, ib), err_msg=f"{n}[{ib}]")
+    finally:
+        for g in (ga, gb, gc):
+            g.close()
