@@ -96,3 +96,9 @@ class Stream:
         if self.handle:
             hip().hipStreamDestroy(self.handle)
             self.handle = None
+
+
+def copy_in(ptr, host):
+    """Host array to a device address of somebody else's."""
+    host = np.ascontiguousarray(host, dtype=np.float64)
+    _chk(hip().hipMemcpy(ptr, host.ctypes.data, host.nbytes, H2D), "hipMemcpy H2D")

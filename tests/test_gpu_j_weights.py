@@ -6,6 +6,7 @@ import pytest
 from mpcns_mercury_amd import cases
 from mpcns_mercury_amd.hip import Mercury
 
+import hipmem
 import restart_format as rf
 
 pytestmark = pytest.mark.gpu
@@ -35,17 +36,19 @@ def test_factors_give_the_stored_weights_bits():
 @pytest.mark.parametrize("how", ["upload", "graph", "address"])
 def test_written_weights_are_used(field, how):
     """After a caller writes the weights (or an edge vector, which leaves the
-    weights as they are), and after it has asked for the address of either, the
+    weights as they are), by an upload or at the address it has asked for, the
     stored weights are the ones that count, also in a step captured before."""
     g = Mercury(_case())
     g.prepare()
+    g.step(2)  # J starts at zero
     if how == "graph":
         g.graph_capture(0)
+    before = _jcell(g)[1]
+    w = g.get(field, 1)
+    w[1] *= 1.5
     if how == "address":
-        g.field_device(field, 1, 1)
+        hipmem.copy_in(g.field_device(field, 1, 1), w[1])
     else:
-        w = g.get(field, 1)
-        w[1] *= 1.5
         g.set(field, 1, w)
     if how == "graph":
         g.graph_launch(1)
@@ -56,6 +59,8 @@ def test_written_weights_are_used(field, how):
         a, own = _jcell(g), Ellipsis
     g.op("jcell")
     np.testing.assert_array_equal(a[1][own], g.get("J_cell", 1)[own])
+    if how != "graph":
+        assert (a[1] != before).any() == (field == "Jcell_from_Jedge_w")
     g.close()
 
 

@@ -136,3 +136,43 @@ def test_resistive_shell_mixed_form(oracle_mod):
     finally:
         g.close()
 
+
+
+def test_solve_of_more_unknowns_than_threads(oracle_mod):
+    """Above 2048 x 256 = 524 288 unknowns a thread of the CG kernels takes more than
+    one, the last trip of some none.  The solution of one solve from the oracle's
+    state, with some 36 iterations, so both scalars of r.z are used many times.
+
+    Bound: both sides stop at a relative residual of 1e-10; 36 iterations to there
+    mean a condition number of about (2 * 36 / ln(2e10))^2 = 9, so each solution is
+    within about 1e-9 of the exact one."""
+    case = cases.make_resistive_shell(scale=0.22, species=2, inver_Rem=0.5)
+    print(f"[case] {case.name} solve of many unknowns", flush=True)
+    g = Mercury(case)
+    o = oracle_mod.Oracle(case)
+    try:
+        g.prepare()
+        o.prepare()
+        o.step(2)
+        for name in ["U_H", "U_Na"] + [f + s for f in ("B", "Eres", "J") for s in AX] + ["B_cell", "Bind_cell", "J_cell"]:
+            for ib in range(case.nb):
+                g.set(name, ib, o.get(name, ib))
+        dt = o.timestep()
+        B0 = {(s, ib): o.get("B" + s, ib) for s in AX for ib in range(case.nb)}
+        g.op("res_solve", dt)
+        its, _ = o.res_solve(dt)
+        n, gits, grel = g.resist_stats()
+        print(f"[res] unknowns={n} its={gits} rel={grel:.2e}; oracle its={its}", flush=True)
+        assert n > 2048 * 256 and n % 256 and gits > 20 and grel <= 1e-10
+        for s in AX:
+            scale = max(np.abs(o.get("Eres" + s, ib)).max() for ib in range(case.nb))
+            assert scale > 0.0
+            for ib in range(case.nb):
+                assert np.abs(g.get("Eres" + s, ib) - o.get("Eres" + s, ib)).max() <= 1e-8 * scale, s
+        dscale = max(np.abs(o.get("B" + s, ib) - B0[s, ib]).max() for s in AX for ib in range(case.nb))
+        assert dscale > 0.0
+        for s in AX:
+            for ib in range(case.nb):
+                assert np.abs(g.get("B" + s, ib) - o.get("B" + s, ib)).max() <= 1e-7 * dscale, s
+    finally:
+        g.close()
