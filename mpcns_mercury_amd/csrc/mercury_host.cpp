@@ -1198,12 +1198,15 @@ public:
     // fill the chip several times over; the kernel keeps two waves per SIMD in
     // FP64 and three in the mixed form, and with fewer than four rounds of them
     // the last round and the longer serial chain cost more.  Measured at 4, 2, 1
-    // cells: 2.53 M cells FP64 360, 367, 387 us and mixed 273, 271, 281; 546 k
-    // cells 120, 107, 105 and 83, 75, 68; 48^3 34, 20, 19; 12x10x8 26, 15, 10.
+    // cells: 15.4 M cells FP64 2155, 2241, 2404 us and mixed 1465, 1481, 1629; 10.4 M
+    // 1381, 1443, 1578 and 985, 1010, 1090; 2.53 M 360, 367, 387 and 273, 271, 281;
+    // 546 k 120, 107, 105 and 83, 75, 68; 48^3 34, 20, 19; 12x10x8 26, 15, 10.  With
+    // three species: 18.9 M 3435, 3590, 3800 and 2239, 2302, 2525; 4.1 M 779, 800, 830
+    // and 553, 552, 590; 2.53 M 505, 512, 534 and 364, 359, 380; 518 k 147, 119, 111
+    // and 86, 81, 71.
     int auto_march() const {
         const long long need = 4LL * simds * (form == 2 ? 3 : 2);
         for (int L : {4, 2}) {
-            if (L == 4 && form == 2 && nspecies() > 2) continue;  // 868 k cells: 145, 139, 161 us at 1, 2, 4
             long long waves = 0;
             for (const MercBlk &k : F->blk) waves += (long long)((k.m[0] + L - 1) / L) * k.m[1] * k.m[2];
             if (waves / 64 >= need) return L;

@@ -64,3 +64,17 @@ def test_shared_edges_take_mean_and_hall(oracle_mod, name):
                     np.testing.assert_array_equal(g.get(n, ib)[own], o.get(n, ib)[own], err_msg=f"{n}[{ib}]")
     finally:
         g.close()
+
+
+def test_flux_shape_of_a_large_context_of_three_species():
+    """Four cells per thread where their waves fill the chip four times over, whatever
+    the number of species (3.2 M cells in the mixed form: 12 600 waves of 12 288)."""
+    case = cases.make_shell(blocks=((160, 140, 144),), he=True)
+    print(f"[case] {case.name} flux shape", flush=True)
+    g = Mercury(case)
+    try:
+        assert g.flux_shape() == (0, 4)
+        g.set_form(2)
+        assert g.flux_shape() == (0, 4)
+    finally:
+        g.close()
