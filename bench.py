@@ -73,7 +73,9 @@ ALGO_BYTES = {
     "jedge": 8 * (3 + 3 + 3 + 3),
     # J (3) + W_j (36) read, J_cell (3) written
     "jcell": 8 * (3 + 36 + 3),
-    # J (3) + inverse 3x3 matrix of the weights (9) + dr (9) read, J_cell (3) written
+    # J (3) + inverse 3x3 matrix of the weights (9) + dr (9) read, J_cell (3) written.  The
+    # mixed form reads 36 weights in FP32 instead, 8 * (3 + 3) + 4 * 36: the same sum.  (A
+    # context whose caller has written weights or dr reads jcell's 36 in FP64.)
     "jcell_t": 8 * (3 + 9 + 9 + 3),
     # U_s (10) + B_cell (3) + JD (9) + Jac (1)
     "timestep": 8 * (10 + 3 + 9 + 1),

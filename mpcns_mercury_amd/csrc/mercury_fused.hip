@@ -548,8 +548,8 @@ __global__ void __launch_bounds__(256) k_rhs_tile(const MercRange R, const MercB
 // without spilling, four in FP64 (five and six spill: 474 us), six in the mixed
 // form with two species, four with three.
 // ENS: an ensemble context (per-block Hall coefficient and per-run dt); a
-// one-run context takes both from the kernel arguments and keeps every
-// register of the six-wave budget for the body.
+// one-run context takes both from the kernel arguments and keeps the registers
+// of that budget for the body.
 template <bool MIX, int NS, bool ENS>
 __global__ void __attribute__((amdgpu_waves_per_eu(MIX ? (NS == 2 ? 6 : 4) : 4))) k_cell_end(const MercRange R, const MercBlk *__restrict__ B, double *const *__restrict__ F_,
                            const float *const *__restrict__ G_, const MercPhys P, unsigned long long *__restrict__ dt_bits,
